@@ -94,6 +94,12 @@ StepParams make_step(double dt, const double* DCr, const double* DNb, const doub
   }
   for (int i = 0; i < 2; i++) P.k[i] *= scale;
   for (int i = 0; i < 9; i++) P.m[i] = mask[i] / scale;
+  // opposite pairs first, then the centre: exactly zero for square cells
+  const double sum = (((P.m[1] + P.m[7]) + (P.m[3] + P.m[5])) +
+                      ((P.m[0] + P.m[8]) + (P.m[2] + P.m[6]))) + P.m[4];
+  P.qs[0] = P.qCr[2] * sum;
+  P.qs[1] = P.qNb[2] * sum;
+  for (int i = 0; i < 2; i++) P.w2[i] = 2.0 * P.w[i];
   for (int c = 0; c < 2; c++) {
     P.xoff[c] = xoff ? xoff[c] : 0.0;
     P.xe_g[c] = XE[0][c] - P.xoff[c];

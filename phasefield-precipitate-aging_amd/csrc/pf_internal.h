@@ -14,9 +14,10 @@ namespace pf {
 // The gamma fictitious composition x_g = xe_g + A_g mu is linear in the
 // potential mu, and so is the Laplacian, so the Cahn-Hilliard update
 // x' = x + dt D lap(x_g) (src/discretization.cu:859-863) is
-//   x_Cr' = x_Cr + lap(q_Cr),  q_Cr = qCr[0] mu0 + qCr[1] mu1 + qCr[2]
-// with q_Cr = dt (D_CrCr x_g,Cr + D_CrNb x_g,Nb), and likewise for Nb.  The
-// Allen-Cahn update (src/discretization.cu:888-942) is
+//   x_Cr' = x_Cr + qCr[0] lap(mu0) + qCr[1] lap(mu1) + qs[0]
+// with dt (D_CrCr x_g,Cr + D_CrNb x_g,Nb) = qCr[0] mu0 + qCr[1] mu1 + qCr[2],
+// and likewise for Nb; qs = q[2] lap(1) is zero for a mask that sums to zero.
+// The Allen-Cahn update (src/discretization.cu:888-942) is
 //   phi' = phi + u (G(mu) u + w (2 phi - 1)) - c phi phi_o^2 + k lap(phi)
 // with u = phi (1 - phi), p'(phi) = 30 u^2, phi (phi - 1)(2 phi - 1) = -u (2 phi - 1)
 // and G = 30 dt L dOmega = g[0] mu0^2 + g[1] mu0 mu1 + g[2] mu1^2 + g[3] mu0 + g[4] mu1.
@@ -36,7 +37,9 @@ namespace pf {
 struct StepParams {
   double qCr[3], qNb[3];  // scale * dt * (D row) . (A_gamma mu + xe_gamma)
   double g[2][5];         // 30 dt L * grand-potential difference  (delta, Laves)
+  double qs[2];           // qCr[2], qNb[2] times the sum of m
   double w[2];            // 2 omega dt L
+  double w2[2];           // 2 w
   double c[2];            // 2 alpha dt L
   double k[2];            // scale * kappa dt L
   double m[9];            // 3x3 Laplacian mask / scale, row-major (y-1, y, y+1)

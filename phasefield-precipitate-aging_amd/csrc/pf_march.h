@@ -6,7 +6,7 @@
 // One wave64 owns a strip of 64 columns (62 output columns + one halo column
 // each side) and marches down a chunk of rows.  Each lane keeps a three-row
 // window (y-1, y, y+1) of what the stencil needs -- phi_delta, phi_Laves and
-// the composition potentials q = dt D x_gamma -- in registers, so each cell
+// the two diffusion potentials mu -- in registers, so each cell
 // is loaded once per strip and its KKS solve is done once.  x-neighbours come
 // from adjacent lanes through DPP wave shifts (no LDS round trip).  Loads run DEPTH
 // rows ahead of the row being computed (a register ring), so a wave keeps
@@ -25,6 +25,12 @@
 
 #include "pf_internal.h"
 #include "pf_thermo.h"
+
+// Every fused multiply-add of the step is written as fma(): the kernels that
+// inline this arithmetic (one to four steps per launch, plain and batched) must
+// give the same bits, and the compiler's own contraction depends on what it
+// sees around an expression.
+#pragma clang fp contract(off)
 
 namespace pf {
 
@@ -83,11 +89,10 @@ __device__ __forceinline__ double from_right(double v) {
 
 struct Point {       // what the neighbours of a cell need
   double pd, pl;     // phase fields
-  double qCr, qNb;   // dt D x_gamma: the Cahn-Hilliard update is x' = x + lap(q)
+  double mu0, mu1;   // common diffusion potential
 };
 struct Centre {      // extra state of a cell when it is the stencil centre
   double xCr, xNb;   // compositions as stored (x - StepParams::xoff)
-  double mu0, mu1;   // common diffusion potential
 };
 template <typename T>
 struct Raw {
@@ -125,17 +130,14 @@ __device__ __forceinline__ void store_row(T* oCr, T* oNb, T* opd, T* opl, size_t
   st_at(opl, row_bytes, lane_bytes, (T)d);
 }
 
-// 1/d to within an ulp or so: hardware reciprocal and two Newton steps (the
-// refinement an IEEE division does before its final rounding correction).
-// Measured on 4M random doubles over 200 binades: the hardware reciprocal
-// alone is good to 2^-24.4, one step leaves results up to 2.2e-15 relative
-// off the correctly rounded 1/d, two give it on every input.
+// 1/d to within an ulp or so: hardware reciprocal r and one third-order step
+// r (1 + e + e^2), e = 1 - d r.  Measured on 4M random doubles over 200
+// binades, the hardware reciprocal is good to 2^-24.4, so the e^3 left out is
+// below 2^-73; a Newton step (r + r e) leaves up to 2.2e-15 relative.
 __device__ __forceinline__ double recip(double d) {
-  double r = __builtin_amdgcn_rcp(d);
-  double e = fma(-d, r, 1.0);
-  r = fma(r, e, r);
-  e = fma(-d, r, 1.0);
-  return fma(r, e, r);
+  const double r = __builtin_amdgcn_rcp(d);
+  const double e = fma(-d, r, 1.0);
+  return fma(r, fma(e, e, e), r);
 }
 // One Newton step (relative error <= 2.2e-15): for FP32 storage, whose every
 // stored value is rounded to 2^-24 relative, so the second step changes no
@@ -157,8 +159,8 @@ __device__ __forceinline__ double p_interp6(double x) {
 // KKS solve of a cell (src/parabola625.cu:245-297 restated): with
 // p_gamma = 1 - p_delta - p_Laves eliminated, M = A_g + p_d (A_d - A_g) +
 // p_l (A_l - A_g) and r = x - xe_g - p_d (xe_d - xe_g) - p_l (xe_l - xe_g);
-// mu = M^-1 r, and the neighbours need q = dt D x_g, x_g = xe_g + A_g mu
-// (linear in mu; coefficients in StepParams).  The constants here carry the
+// mu = M^-1 r, and the neighbours need mu (x_g = xe_g + A_g mu is linear in
+// it).  The constants here carry the
 // factor 6 of p_interp6.  x - xe_g is formed from the stored composition and
 // P.xe_g (xe_g less the storage offset).
 constexpr double DA_DEL[3] = {6.0 * (A[1][0] - A[0][0]), 6.0 * (A[1][1] - A[0][1]),
@@ -168,33 +170,60 @@ constexpr double DA_LAV[3] = {6.0 * (A[2][0] - A[0][0]), 6.0 * (A[2][1] - A[0][1
 constexpr double DXE_DEL[2] = {6.0 * (XE[1][0] - XE[0][0]), 6.0 * (XE[1][1] - XE[0][1])};
 constexpr double DXE_LAV[2] = {6.0 * (XE[2][0] - XE[0][0]), 6.0 * (XE[2][1] - XE[0][1])};
 
+// Addends of FMAs whose multiplicand is a constant too.  A VOP3 instruction
+// reads one scalar register pair at most, so one of the two constants has to
+// be in vector registers; keeping these there for the whole march saves a
+// move before each use (the empty asm stops the compiler from rebuilding them
+// from scalars every time).
+struct Addends {
+  double A[3];          // A_gamma
+  double qs[2];         // StepParams::qs
+  double g3[2], g4[2];  // StepParams::g[.][3], [4]
+  double w[2];          // -StepParams::w
+};
+__device__ __forceinline__ double in_vgpr(double x) {
+  asm("" : "+v"(x));
+  return x;
+}
+__device__ __forceinline__ Addends addends(const StepParams& P) {
+  Addends a;
+#pragma unroll
+  for (int i = 0; i < 3; i++) a.A[i] = in_vgpr(A[0][i]);
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    a.qs[i] = in_vgpr(P.qs[i]);
+    a.g3[i] = in_vgpr(P.g[i][3]);
+    a.g4[i] = in_vgpr(P.g[i][4]);
+    a.w[i] = in_vgpr(-P.w[i]);
+  }
+  return a;
+}
+
 template <typename T>
-__device__ __forceinline__ void derive(const StepParams& P, const Raw<T>& r, Point& v,
-                                       Centre& c) {
+__device__ __forceinline__ void derive(const StepParams& P, const Addends& ad, const Raw<T>& r,
+                                       Point& v, Centre& c) {
   v.pd = (double)r.pd;
   v.pl = (double)r.pl;
   c.xCr = (double)r.cr;
   c.xNb = (double)r.nb;
   const double pD = p_interp6(v.pd);
   const double pL = p_interp6(v.pl);
-  const double M0 = fma(pD, DA_DEL[0], fma(pL, DA_LAV[0], A[0][0]));
-  const double M1 = fma(pD, DA_DEL[1], fma(pL, DA_LAV[1], A[0][1]));
-  const double M2 = fma(pD, DA_DEL[2], fma(pL, DA_LAV[2], A[0][2]));
+  const double M0 = fma(pD, DA_DEL[0], fma(pL, DA_LAV[0], ad.A[0]));
+  const double M1 = fma(pD, DA_DEL[1], fma(pL, DA_LAV[1], ad.A[1]));
+  const double M2 = fma(pD, DA_DEL[2], fma(pL, DA_LAV[2], ad.A[2]));
   const double r0 = fma(-pD, DXE_DEL[0], fma(-pL, DXE_LAV[0], c.xCr - P.xe_g[0]));
   const double r1 = fma(-pD, DXE_DEL[1], fma(-pL, DXE_LAV[1], c.xNb - P.xe_g[1]));
   const double det = fma(M0, M2, -(M1 * M1));
   const double inv = sizeof(T) == sizeof(float) ? recip1(det) : recip(det);
-  c.mu0 = fma(M2, r0, -(M1 * r1)) * inv;
-  c.mu1 = fma(M0, r1, -(M1 * r0)) * inv;
-  v.qCr = fma(P.qCr[0], c.mu0, fma(P.qCr[1], c.mu1, P.qCr[2]));
-  v.qNb = fma(P.qNb[0], c.mu0, fma(P.qNb[1], c.mu1, P.qNb[2]));
+  v.mu0 = fma(M2, r0, -(M1 * r1)) * inv;
+  v.mu1 = fma(M0, r1, -(M1 * r0)) * inv;
 }
 
 __device__ __forceinline__ Point shift_left(const Point& a) {
-  return Point{from_left(a.pd), from_left(a.pl), from_left(a.qCr), from_left(a.qNb)};
+  return Point{from_left(a.pd), from_left(a.pl), from_left(a.mu0), from_left(a.mu1)};
 }
 __device__ __forceinline__ Point shift_right(const Point& a) {
-  return Point{from_right(a.pd), from_right(a.pl), from_right(a.qCr), from_right(a.qNb)};
+  return Point{from_right(a.pd), from_right(a.pl), from_right(a.mu0), from_right(a.mu1)};
 }
 
 // Nucleation of one cell from its new values (centre-only scan; the caller
@@ -253,19 +282,19 @@ __device__ __forceinline__ void laplacians(const double* m, const Point& S, cons
                                            const Point& C, const Point& E, const Point& Nn,
                                            const Point& SW, const Point& SE, const Point& NW,
                                            const Point& NE, double lap[4]) {
-  const double s[4] = {S.pd, S.pl, S.qCr, S.qNb};
-  const double w[4] = {W.pd, W.pl, W.qCr, W.qNb};
-  const double c[4] = {C.pd, C.pl, C.qCr, C.qNb};
-  const double e[4] = {E.pd, E.pl, E.qCr, E.qNb};
-  const double n[4] = {Nn.pd, Nn.pl, Nn.qCr, Nn.qNb};
+  const double s[4] = {S.pd, S.pl, S.mu0, S.mu1};
+  const double w[4] = {W.pd, W.pl, W.mu0, W.mu1};
+  const double c[4] = {C.pd, C.pl, C.mu0, C.mu1};
+  const double e[4] = {E.pd, E.pl, E.mu0, E.mu1};
+  const double n[4] = {Nn.pd, Nn.pl, Nn.mu0, Nn.mu1};
 #pragma unroll
   for (int f = 0; f < 4; f++) {
     double v;
     if (NINE) {
-      const double sw[4] = {SW.pd, SW.pl, SW.qCr, SW.qNb};
-      const double se[4] = {SE.pd, SE.pl, SE.qCr, SE.qNb};
-      const double nw[4] = {NW.pd, NW.pl, NW.qCr, NW.qNb};
-      const double ne[4] = {NE.pd, NE.pl, NE.qCr, NE.qNb};
+      const double sw[4] = {SW.pd, SW.pl, SW.mu0, SW.mu1};
+      const double se[4] = {SE.pd, SE.pl, SE.mu0, SE.mu1};
+      const double nw[4] = {NW.pd, NW.pl, NW.mu0, NW.mu1};
+      const double ne[4] = {NE.pd, NE.pl, NE.mu0, NE.mu1};
       v = m[0] * sw[f];
       v = fma(m[1], s[f], v);
       v = fma(m[2], se[f], v);
@@ -287,25 +316,31 @@ __device__ __forceinline__ void laplacians(const double* m, const Point& S, cons
 // Cahn-Hilliard (src/discretization.cu:859-863) and Allen-Cahn
 // (src/discretization.cu:888-942) with the closed-form grand-potential
 // difference at the solved potential, as the quadratic form of StepParams.
-// The composition increment lap(q) is formed on its own and added to x once,
-// as the reference adds dt D lap(x_g): where the increment is ~0 (the
-// uniform matrix) x comes back unchanged, so rounding adds no drift there.
-__device__ __forceinline__ void update_cell(const StepParams& P, const double lap[4],
-                                            const Point& cur, const Centre& cc, double& nCr,
-                                            double& nNb, double& npd, double& npl) {
-  nCr = cc.xCr + lap[2];
-  nNb = cc.xNb + lap[3];
+// The composition increment is formed on its own from the Laplacians of the
+// potential and added to x once, as the reference adds dt D lap(x_g): where
+// the increment is ~0 (the uniform matrix) x comes back unchanged, so rounding
+// adds no drift there.  The kernels are bound by the FP64 operations they
+// issue, so the sums are nested to take the fewest: the Laplacians of mu (not
+// of dt D x_gamma) save the two products of q per cell and two doubles of
+// state per level, the quadratic form is evaluated in two brackets with no
+// squares, and u (G u + w (2 phi - 1)) and c phi phi_o^2 are folded into
+// FMAs: 33 operations after the Laplacians, 41 with the terms written out.
+__device__ __forceinline__ void update_cell(const StepParams& P, const Addends& ad,
+                                            const double lap[4], const Point& cur, const Centre& cc, double& nCr, double& nNb,
+                                            double& npd, double& npl) {
+  nCr = cc.xCr + fma(P.qCr[0], lap[2], fma(P.qCr[1], lap[3], ad.qs[0]));
+  nNb = cc.xNb + fma(P.qNb[0], lap[2], fma(P.qNb[1], lap[3], ad.qs[1]));
   const double fd = cur.pd, fl = cur.pl;
-  const double m00 = cc.mu0 * cc.mu0, m01 = cc.mu0 * cc.mu1, m11 = cc.mu1 * cc.mu1;
-  const double Gd = fma(P.g[0][0], m00, fma(P.g[0][1], m01, fma(P.g[0][2], m11,
-                    fma(P.g[0][3], cc.mu0, P.g[0][4] * cc.mu1))));
-  const double Gl = fma(P.g[1][0], m00, fma(P.g[1][1], m01, fma(P.g[1][2], m11,
-                    fma(P.g[1][3], cc.mu0, P.g[1][4] * cc.mu1))));
+  const double Gd = fma(cur.mu0, fma(P.g[0][0], cur.mu0, fma(P.g[0][1], cur.mu1, ad.g3[0])),
+                        cur.mu1 * fma(P.g[0][2], cur.mu1, ad.g4[0]));
+  const double Gl = fma(cur.mu0, fma(P.g[1][0], cur.mu0, fma(P.g[1][1], cur.mu1, ad.g3[1])),
+                        cur.mu1 * fma(P.g[1][2], cur.mu1, ad.g4[1]));
   const double ud = fma(-fd, fd, fd), ul = fma(-fl, fl, fl);  // phi (1 - phi)
-  const double td = ud * fma(ud, Gd, P.w[0] * fma(2.0, fd, -1.0));
-  const double tl = ul * fma(ul, Gl, P.w[1] * fma(2.0, fl, -1.0));
-  npd = fma(-P.c[0] * fd, fl * fl, fma(P.k[0], lap[0], fd) + td);
-  npl = fma(-P.c[1] * fl, fd * fd, fma(P.k[1], lap[1], fl) + tl);
+  const double td = fma(ud, Gd, fma(P.w2[0], fd, ad.w[0]));
+  const double tl = fma(ul, Gl, fma(P.w2[1], fl, ad.w[1]));
+  const double z = fd * fl;
+  npd = fma(-(P.c[0] * z), fl, fma(ud, td, fma(P.k[0], lap[0], fd)));
+  npl = fma(-(P.c[1] * z), fd, fma(ul, tl, fma(P.k[1], lap[1], fl)));
 }
 
 template <typename T>
@@ -377,6 +412,7 @@ __device__ __forceinline__ void march(
     load_row(r, iCr, iNb, ipd, ipl, (size_t)(1 + bc_map<BC>(y, Ny)) * row_b, in_lane);
   };
 
+  const Addends ad = addends(P);
   // window slots (row y0 + k - 1 + 3j lives in slot k % 3 pattern below)
   Point win[3];
   Centre cen[3];
@@ -386,9 +422,9 @@ __device__ __forceinline__ void march(
   {
     Raw<T> r;
     load(r, y0 - 1);
-    derive<T>(P, r, win[2], cen[2]);
+    derive<T>(P, ad, r, win[2], cen[2]);
     load(r, y0);
-    derive<T>(P, r, win[0], cen[0]);
+    derive<T>(P, ad, r, win[0], cen[0]);
   }
 #pragma unroll
   for (int j = 0; j < DEPTH; j++) load(ring[j], min(y0 + 1 + j, y1));
@@ -407,7 +443,7 @@ __device__ __forceinline__ void march(
       if (y >= y1) return;
       const int ps = (k + 2) % 3, cs = k % 3, ns = (k + 1) % 3;
       const int rs = k % DEPTH;
-      derive<T>(P, ring[rs], win[ns], cen[ns]);
+      derive<T>(P, ad, ring[rs], win[ns], cen[ns]);
       load(ring[rs], min(y + 1 + DEPTH, y1));
 
       Point W, E;
@@ -425,7 +461,7 @@ __device__ __forceinline__ void march(
                        winE[ns], lap);
 
       double nCr, nNb, npd, npl;
-      update_cell(P, lap, win[cs], cen[cs], nCr, nNb, npd, npl);
+      update_cell(P, ad, lap, win[cs], cen[cs], nCr, nNb, npd, npl);
 
       const int py = 1 + y;
       if (NUC && out_lane) {
@@ -473,12 +509,10 @@ __device__ __forceinline__ void march(
 // t % 3; the first 2K iterations (the prologue) are unrolled at compile time.
 //
 // With a window array `lw` in LDS (LW = true, the four-step kernel), each
-// level's row also goes to LDS at the end of the iteration that computed it
-// and comes back from there two iterations later as the row behind: the
-// register windows then hold two live rows per level, not three, which is
-// what lets four levels fit in the registers of two waves per SIMD.  Each
-// lane reads back only what it wrote itself, so no barrier is needed.  The
-// array holds 2 slots (iteration parity) x K levels x 4 values x 64 lanes.
+// level's centre row goes to LDS at the end of an iteration and comes back at
+// the next as the row behind: the register windows then hold two live rows
+// per level, not three.  Each lane reads back only what it wrote itself, so no
+// barrier is needed.  The array holds K levels x 4 values x 64 lanes.
 //
 // The intermediate levels are exactly what one-step launches would have
 // stored: values are rounded to the storage type before the next level uses
@@ -504,7 +538,6 @@ __device__ __forceinline__ void marchk_impl(
     T* __restrict__ opl, int Nx, int Ny, int pitch, int strip, int chunk, int rows,
     const StepParams& P, LdsPtr lw) {
   static_assert(K >= 2 && K <= 4, "two to four steps per pass");
-  static_assert(UNROLL % 2 == 0, "the LDS slot is the iteration parity");
   static_assert(UNROLL % DEPTH == 0, "ring depth must divide the unroll factor");
   // SW output columns per strip (64 - 2K, or fewer where the strips are laid
   // out for a deeper march); lanes K .. K+SW-1 store
@@ -528,25 +561,26 @@ __device__ __forceinline__ void marchk_impl(
     load_row(r, iCr, iNb, ipd, ipl, (size_t)(1 + bc_map<BC>(y, Ny)) * row_b, in_lane);
   };
   const double* m = P.m;
+  const Addends ad = addends(P);
 
   // windows: level l (0 = old fields) row of iteration t in slot t % 3
   Point win[K][3];
   Centre cen[K][3];
   Raw<T> ring[DEPTH];
 
-  // LDS copy of level l's row of an iteration of parity `slot`
-  auto put = [&](int l, int slot, const Point& v) {
-    LdsPtr q = lw + ((l * 2 + slot) * 4) * WAVE + lane;
+  // LDS copy of the row of level l that is behind at the next iteration
+  auto put = [&](int l, const Point& v) {
+    LdsPtr q = lw + (l * 4) * WAVE + lane;
     q[0] = v.pd;
     q[WAVE] = v.pl;
-    q[2 * WAVE] = v.qCr;
-    q[3 * WAVE] = v.qNb;
+    q[2 * WAVE] = v.mu0;
+    q[3 * WAVE] = v.mu1;
   };
-  // level l's row behind at iteration t (slot sb of the window; in LDS, the
-  // row stored at iteration t - 2, of the same parity)
-  auto behind = [&](int l, int sb, int par) -> Point {
+  // level l's row behind (slot sb of the window; in LDS, the centre row of
+  // the iteration before)
+  auto behind = [&](int l, int sb) -> Point {
     if constexpr (LW) {
-      const LdsPtr q = lw + ((l * 2 + par) * 4) * WAVE + lane;
+      const LdsPtr q = lw + (l * 4) * WAVE + lane;
       return Point{q[0], q[WAVE], q[2 * WAVE], q[3 * WAVE]};
     } else {
       return win[l][sb];
@@ -561,32 +595,33 @@ __device__ __forceinline__ void marchk_impl(
     double lap[4];
     laplacians<false>(m, Sth, W, C, E, Nth, Sth, Sth, Nth, Nth, lap);
     double n0, n1, n2, n3;
-    update_cell(P, lap, C, cc, n0, n1, n2, n3);
+    update_cell(P, ad, lap, C, cc, n0, n1, n2, n3);
     Raw<T> r;
     r.cr = (T)n0;
     r.nb = (T)n1;
     r.pd = (T)n2;
     r.pl = (T)n3;
-    derive<T>(P, r, v, c);
+    derive<T>(P, ad, r, v, c);
   };
 
   // Levels 1..K-1 at iteration t (slots are compile-time in both callers):
   // level l computes row y0-K+t-l.
-  auto middle_levels = [&](int sa, int sc, int sb, int lmax_active, int par) {
+  auto middle_levels = [&](int sa, int sc, int sb, int lmax_active) {
 #pragma unroll
     for (int l = 1; l < K; l++) {
       if (l > lmax_active) break;
-      level_up(behind(l - 1, sb, par), win[l - 1][sc], cen[l - 1][sc], win[l - 1][sa],
-               win[l][sa], cen[l][sa]);
+      level_up(behind(l - 1, sb), win[l - 1][sc], cen[l - 1][sc], win[l - 1][sa], win[l][sa],
+               cen[l][sa]);
     }
   };
-  // end of iteration t: the rows of the active levels to LDS
-  auto put_rows = [&](int sa, int lmax_active, int par) {
+  // end of iteration t: the centre rows of the levels active before it to
+  // LDS, over the rows behind that the iteration has read
+  auto put_rows = [&](int sc, int levels) {
     if constexpr (LW) {
 #pragma unroll
       for (int l = 0; l < K; l++) {
-        if (l > lmax_active) break;
-        put(l, par, win[l][sa]);
+        if (l >= levels) break;
+        put(l, win[l][sc]);
       }
     }
   };
@@ -603,15 +638,14 @@ __device__ __forceinline__ void marchk_impl(
 #pragma unroll
     for (int t = 0; t < 2 * K; t++) {
       const int sa = t % 3, sc = (t + 2) % 3, sb = (t + 1) % 3;
-      derive<T>(P, pro[t], win[0][sa], cen[0][sa]);
+      derive<T>(P, ad, pro[t], win[0][sa], cen[0][sa]);
       // level l is active from iteration 2l on
-      middle_levels(sa, sc, sb, t / 2, t % 2);
-      put_rows(sa, t / 2, t % 2);
+      middle_levels(sa, sc, sb, t / 2);
+      put_rows(sc, (t + 1) / 2);
     }
   }
 
-  // ---- main loop: iteration t = 2K + i, output row y = y0 + i (t and k
-  // have the same parity: 2K and UNROLL are even)
+  // ---- main loop: iteration t = 2K + i, output row y = y0 + i
   for (int ib = 0;; ib += UNROLL) {
 #pragma unroll
     for (int k = 0; k < UNROLL; k++) {
@@ -619,23 +653,23 @@ __device__ __forceinline__ void marchk_impl(
       const int y = y0 + ib + k;
       const int sa = (2 * K + k) % 3, sc = (2 * K + k + 2) % 3, sb = (2 * K + k + 1) % 3;
       const int rs = k % DEPTH;
-      derive<T>(P, ring[rs], win[0][sa], cen[0][sa]);  // old row y + K
+      derive<T>(P, ad, ring[rs], win[0][sa], cen[0][sa]);  // old row y + K
       load(ring[rs], min(y + K + DEPTH, y_last));
-      middle_levels(sa, sc, sb, K - 1, k % 2);
+      middle_levels(sa, sc, sb, K - 1);
       // level K: row y from level K-1's rows y-1 (behind), y, y+1 (ahead)
-      const Point Sth = behind(K - 1, sb, k % 2);
+      const Point Sth = behind(K - 1, sb);
       const Point& C = win[K - 1][sc];
       const Point& Nth = win[K - 1][sa];
       const Point W = shift_left(C), E = shift_right(C);
       double lap[4];
       laplacians<false>(m, Sth, W, C, E, Nth, Sth, Sth, Nth, Nth, lap);
       double nCr, nNb, npd, npl;
-      update_cell(P, lap, C, cen[K - 1][sc], nCr, nNb, npd, npl);
+      update_cell(P, ad, lap, C, cen[K - 1][sc], nCr, nNb, npd, npl);
       if (out_lane) {
         store_row(oCr, oNb, opd, opl, (size_t)(1 + y) * row_b, out_lane_b, nCr, nNb, npd, npl);
         store_ghost_images<T, BC>(oCr, oNb, opd, opl, gx, y, Nx, Ny, pitch, nCr, nNb, npd, npl);
       }
-      put_rows(sa, K - 1, k % 2);
+      put_rows(sc, K);
     }
   }
 }
@@ -651,3 +685,5 @@ __device__ __forceinline__ void marchk(
 }
 
 }  // namespace pf
+
+#pragma clang fp contract(fast)  // the compiler's default for device code

@@ -118,9 +118,13 @@ __global__ __launch_bounds__(WAVE * WPB) void stepk_kernel(
                           b / strips, rows, P);
 }
 
-// Four steps: the rows behind of the four levels' windows live in LDS (16 KiB
-// per wave, 64 KiB per block of WPB = 4 waves), which caps the kernel at two
-// blocks, so two waves per SIMD, per CU; the register budget is set to match.
+// Four steps: the rows behind of the four levels' windows live in LDS (8 KiB
+// per wave, 32 KiB per block of WPB = 4 waves); 223 VGPRs allow two waves per
+// SIMD and the register budget is set to match.  At three waves per SIMD (168
+// VGPRs) it spills and takes twice as long.  FP64 4096^2: 326 us per launch
+// on a domain full of particles (380 us before the sums of update_cell were
+// nested and its constant addends kept in vector registers), 75% of it VALU
+// issue.
 template <typename T, int BC, int DEPTH>
 __global__ __launch_bounds__(WAVE * WPB) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void step4_kernel(const T* __restrict__ iCr, const T* __restrict__ iNb,
@@ -128,7 +132,7 @@ void step4_kernel(const T* __restrict__ iCr, const T* __restrict__ iNb,
                   T* __restrict__ oNb, T* __restrict__ opd, T* __restrict__ opl, int Nx, int Ny,
                   int pitch, int strips, int chunks, int rows, int remap, StepParams P) {
   constexpr int K = 4;
-  constexpr int PER_WAVE = K * 2 * 4 * WAVE;  // levels x parity x values x lanes
+  constexpr int PER_WAVE = K * 4 * WAVE;  // levels x values x lanes
   __shared__ double win_lds[WPB * PER_WAVE];
   const int nwaves = strips * chunks;
   const int nblocks = (nwaves + WPB - 1) / WPB;
