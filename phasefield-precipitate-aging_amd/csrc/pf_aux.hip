@@ -59,6 +59,28 @@ NucParams make_nuc(double sigma_del, double sigma_lav, double unit_a, double dx,
   return N;
 }
 
+// Whether the bounds hold that the march's MATRIX and QUIET modes rest on, for
+// up to four steps from |phi| < PHI_MATRIX and |x| < X_MATRIX: one step raises
+// |phi| < TINY at most 16-fold, and the potentials stay small enough that the
+// driving force times TINY is far below one.  In matrix cells mu = H_g (x - xe_g),
+// so a step changes it by at most |H_g| |q| |lap(mu)|.  False for NaN.
+static bool matrix_bounds(const StepParams& P) {
+  const double lm = fabs(P.m[1]) + fabs(P.m[7]) + fabs(P.m[3]) + fabs(P.m[5]) + fabs(P.m[4]);
+  const double h = fmax(fabs(H[0][0]) + fabs(H[0][1]), fabs(H[0][1]) + fabs(H[0][2]));
+  const double q = fmax(fabs(P.qCr[0]) + fabs(P.qCr[1]), fabs(P.qNb[0]) + fabs(P.qNb[1]));
+  const double qs = fmax(fabs(P.qs[0]), fabs(P.qs[1]));
+  double mu = h * (X_MATRIX + 1.0 + fmax(fabs(P.xoff[0]), fabs(P.xoff[1])));
+  for (int step = 0; step < 4; step++) mu = 1.01 * (mu + h * (q * lm * mu + qs + 1e-5));
+  for (int a = 0; a < 2; a++) {
+    const double* g = P.g[a];
+    const double G = (fabs(g[0]) + fabs(g[1]) + fabs(g[2])) * mu * mu +
+                     (fabs(g[3]) + fabs(g[4])) * mu;
+    if (!(G < 0x1p50) || !(fabs(P.c[a]) < 0x1p50) || !(fabs(P.k[a]) * lm + fabs(P.w[a]) < 14.0))
+      return false;
+  }
+  return symmetric_five_point(P.m);
+}
+
 StepParams make_step(double dt, const double* DCr, const double* DNb, const double* kappa,
                      const double* omega, const double* Lmob, double alpha, const double* mask,
                      const double* xoff) {
@@ -102,8 +124,9 @@ StepParams make_step(double dt, const double* DCr, const double* DNb, const doub
   for (int i = 0; i < 2; i++) P.w2[i] = 2.0 * P.w[i];
   for (int c = 0; c < 2; c++) {
     P.xoff[c] = xoff ? xoff[c] : 0.0;
-    P.xe_g[c] = XE[0][c] - P.xoff[c];
+    P.xe_mid[c] = 0.5 * (XE[1][c] + XE[2][c]) - P.xoff[c];
   }
+  P.matrix_ok = matrix_bounds(P) ? 1 : 0;
   return P;
 }
 

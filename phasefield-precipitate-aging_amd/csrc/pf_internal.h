@@ -31,8 +31,8 @@ namespace pf {
 // Stored compositions may be offset: an array holds x - xoff (FP32 storage
 // with xoff near the mean composition keeps 4-5 more bits of the small
 // per-step increments; xoff = 0 otherwise).  The step is offset-invariant but
-// for the residual x - xe_gamma of the KKS solve, so the kernels work on stored
-// values throughout with xe_g = xe_gamma - xoff; only the nucleation test
+// for the residual x - xe of the KKS solve, so the kernels work on stored
+// values throughout with xoff taken off its constant xe_mid; only the nucleation test
 // (which evaluates g and D at x) adds xoff back.
 struct StepParams {
   double qCr[3], qNb[3];  // scale * dt * (D row) . (A_gamma mu + xe_gamma)
@@ -43,9 +43,13 @@ struct StepParams {
   double c[2];            // 2 alpha dt L
   double k[2];            // scale * kappa dt L
   double m[9];            // 3x3 Laplacian mask / scale, row-major (y-1, y, y+1)
-  double xe_g[2];         // xe_gamma - xoff (Cr, Nb)
+  double xe_mid[2];       // (xe_delta + xe_Laves) / 2 - xoff (Cr, Nb)
   double xoff[2];         // composition offset of the stored arrays (Cr, Nb)
+  int matrix_ok;          // the multi-step march may treat matrix rows apart (pf_march.h)
 };
+// What counts as matrix there: phase fields that four steps cannot raise to
+// TINY (2^-56), compositions that keep every product finite.
+constexpr double PHI_MATRIX = 0x1p-72, X_MATRIX = 8.0;
 
 // The masks the folded five-point Laplacian takes (as given by the caller).
 inline bool symmetric_five_point(const double* m) {

@@ -23,6 +23,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "pf_internal.h"
 #include "pf_thermo.h"
 
@@ -53,23 +55,18 @@ __device__ __forceinline__ int xcd_remap(int b, int nb) {
 }
 
 // Interior index map.  No-flux (BC 0): even reflection about the domain
-// faces, period 2n (-1 -> 0, -2 -> 1, n -> n-1, n+1 -> n-2, ...).  At the one
+// faces (-1 -> 0, -2 -> 1, ..., n -> n-1, n+1 -> n-2, ...).  At the one
 // ghost layer (i = -1, n) this is the reference's ghost copy
 // (src/discretization.cu:360-394); deeper halo cells (the multi-step march)
 // are the mirror images that make every intermediate level's halo equal,
-// bit for bit, to the ghost copy of that level (see marchk_impl).  Any i maps
-// into [0, n).  Periodic (BC 1): wrap, for i in [-n, 2n) (values beyond are
-// clamped, unused).
+// bit for bit, to the ghost copy of that level (see marchk_impl).  Periodic
+// (BC 1): wrap.  Both for i in [-n, 2n); any other i maps into [0, n) too
+// (lanes past the last strip's halo, unused).  No division: the march maps a
+// row index per iteration.
 template <int BC>
 __device__ __forceinline__ int bc_map(int i, int n) {
-  if (BC == 0) {
-    const int p = 2 * n;
-    int m = i % p;
-    if (m < 0) m += p;
-    return m < n ? m : p - 1 - m;
-  }
-  if (i < 0) return i + n;
-  if (i >= n) return (i - n) < n ? i - n : n - 1;
+  if (i < 0) return BC == 0 ? min(-1 - i, n - 1) : i + n;
+  if (i >= n) return BC == 0 ? max(2 * n - 1 - i, 0) : ((i - n) < n ? i - n : n - 1);
   return i;
 }
 
@@ -148,27 +145,30 @@ __device__ __forceinline__ double recip1(double d) {
   return fma(r, fma(-d, r, 1.0), r);
 }
 
-// interpolator p(x) = x^3 (6x^2 - 15x + 10), returned divided by 6:
-// x^3 (x (x - 5/2) + 5/3).  The factor 6 is folded into the constants p
-// multiplies (DA_*, DXE_*), which keeps every operation to one constant
-// operand.
-__device__ __forceinline__ double p_interp6(double x) {
-  return (x * x) * x * fma(x, x - 2.5, 5.0 / 3.0);
+// Interpolator p(x) = x^3 (6x^2 - 15x + 10), returned less one half:
+// p - 1/2 = (x - 1/2) (1 + 2u + 6u^2), u = x (1 - x).  The halves are folded
+// into the constants p multiplies.  Five operations, as the power form takes;
+// for |x| < TINY this gives exactly -1/2 (u = x, x - 1/2 and 1 + 2u round to
+// -1/2 and 1), which is what lets matrix cells share one set of coefficients
+// (MatrixCoef).
+constexpr double TINY = 0x1p-56;
+__device__ __forceinline__ double p_less_half(double x) {
+  const double u = fma(-x, x, x);
+  return (x - 0.5) * fma(u, fma(6.0, u, 2.0), 1.0);
 }
 
 // KKS solve of a cell (src/parabola625.cu:245-297 restated): with
-// p_gamma = 1 - p_delta - p_Laves eliminated, M = A_g + p_d (A_d - A_g) +
-// p_l (A_l - A_g) and r = x - xe_g - p_d (xe_d - xe_g) - p_l (xe_l - xe_g);
-// mu = M^-1 r, and the neighbours need mu (x_g = xe_g + A_g mu is linear in
-// it).  The constants here carry the
-// factor 6 of p_interp6.  x - xe_g is formed from the stored composition and
-// P.xe_g (xe_g less the storage offset).
-constexpr double DA_DEL[3] = {6.0 * (A[1][0] - A[0][0]), 6.0 * (A[1][1] - A[0][1]),
-                              6.0 * (A[1][2] - A[0][2])};
-constexpr double DA_LAV[3] = {6.0 * (A[2][0] - A[0][0]), 6.0 * (A[2][1] - A[0][1]),
-                              6.0 * (A[2][2] - A[0][2])};
-constexpr double DXE_DEL[2] = {6.0 * (XE[1][0] - XE[0][0]), 6.0 * (XE[1][1] - XE[0][1])};
-constexpr double DXE_LAV[2] = {6.0 * (XE[2][0] - XE[0][0]), 6.0 * (XE[2][1] - XE[0][1])};
+// p_gamma = 1 - p_delta - p_Laves eliminated and q = p - 1/2,
+// M = M_mid + q_d (A_d - A_g) + q_l (A_l - A_g), M_mid = (A_d + A_l) / 2, and
+// r = x - xe_mid - q_d (xe_d - xe_g) - q_l (xe_l - xe_g), xe_mid = (xe_d + xe_l) / 2
+// less the storage offset (StepParams::xe_mid); mu = M^-1 r, and the
+// neighbours need mu (x_g = xe_g + A_g mu is linear in it).
+constexpr double DA_DEL[3] = {A[1][0] - A[0][0], A[1][1] - A[0][1], A[1][2] - A[0][2]};
+constexpr double DA_LAV[3] = {A[2][0] - A[0][0], A[2][1] - A[0][1], A[2][2] - A[0][2]};
+constexpr double A_MID[3] = {0.5 * (A[1][0] + A[2][0]), 0.5 * (A[1][1] + A[2][1]),
+                             0.5 * (A[1][2] + A[2][2])};
+constexpr double DXE_DEL[2] = {XE[1][0] - XE[0][0], XE[1][1] - XE[0][1]};
+constexpr double DXE_LAV[2] = {XE[2][0] - XE[0][0], XE[2][1] - XE[0][1]};
 
 // Addends of FMAs whose multiplicand is a constant too.  A VOP3 instruction
 // reads one scalar register pair at most, so one of the two constants has to
@@ -176,7 +176,8 @@ constexpr double DXE_LAV[2] = {6.0 * (XE[2][0] - XE[0][0]), 6.0 * (XE[2][1] - XE
 // move before each use (the empty asm stops the compiler from rebuilding them
 // from scalars every time).
 struct Addends {
-  double A[3];          // A_gamma
+  double A[3];          // A_MID
+  double xe[2];         // -StepParams::xe_mid
   double qs[2];         // StepParams::qs
   double g3[2], g4[2];  // StepParams::g[.][3], [4]
   double w[2];          // -StepParams::w
@@ -188,9 +189,10 @@ __device__ __forceinline__ double in_vgpr(double x) {
 __device__ __forceinline__ Addends addends(const StepParams& P) {
   Addends a;
 #pragma unroll
-  for (int i = 0; i < 3; i++) a.A[i] = in_vgpr(A[0][i]);
+  for (int i = 0; i < 3; i++) a.A[i] = in_vgpr(A_MID[i]);
 #pragma unroll
   for (int i = 0; i < 2; i++) {
+    a.xe[i] = in_vgpr(-P.xe_mid[i]);
     a.qs[i] = in_vgpr(P.qs[i]);
     a.g3[i] = in_vgpr(P.g[i][3]);
     a.g4[i] = in_vgpr(P.g[i][4]);
@@ -199,24 +201,38 @@ __device__ __forceinline__ Addends addends(const StepParams& P) {
   return a;
 }
 
+// What the phase fields of a cell determine of its solve: M, 1/det M and the
+// composition-free part t of r = x + t.
+struct Coef {
+  double M0, M1, M2, t0, t1, inv;
+};
 template <typename T>
-__device__ __forceinline__ void derive(const StepParams& P, const Addends& ad, const Raw<T>& r,
-                                       Point& v, Centre& c) {
+__device__ __forceinline__ Coef coefficients(const Addends& ad, double pd, double pl) {
+  const double qD = p_less_half(pd);
+  const double qL = p_less_half(pl);
+  Coef k;
+  k.M0 = fma(qD, DA_DEL[0], fma(qL, DA_LAV[0], ad.A[0]));
+  k.M1 = fma(qD, DA_DEL[1], fma(qL, DA_LAV[1], ad.A[1]));
+  k.M2 = fma(qD, DA_DEL[2], fma(qL, DA_LAV[2], ad.A[2]));
+  k.t0 = fma(-qD, DXE_DEL[0], fma(-qL, DXE_LAV[0], ad.xe[0]));
+  k.t1 = fma(-qD, DXE_DEL[1], fma(-qL, DXE_LAV[1], ad.xe[1]));
+  const double det = fma(k.M0, k.M2, -(k.M1 * k.M1));
+  k.inv = sizeof(T) == sizeof(float) ? recip1(det) : recip(det);
+  return k;
+}
+__device__ __forceinline__ void solve(const Coef& k, const Centre& c, Point& v) {
+  const double r0 = c.xCr + k.t0, r1 = c.xNb + k.t1;
+  v.mu0 = fma(k.M2, r0, -(k.M1 * r1)) * k.inv;
+  v.mu1 = fma(k.M0, r1, -(k.M1 * r0)) * k.inv;
+}
+
+template <typename T>
+__device__ __forceinline__ void derive(const Addends& ad, const Raw<T>& r, Point& v, Centre& c) {
   v.pd = (double)r.pd;
   v.pl = (double)r.pl;
   c.xCr = (double)r.cr;
   c.xNb = (double)r.nb;
-  const double pD = p_interp6(v.pd);
-  const double pL = p_interp6(v.pl);
-  const double M0 = fma(pD, DA_DEL[0], fma(pL, DA_LAV[0], ad.A[0]));
-  const double M1 = fma(pD, DA_DEL[1], fma(pL, DA_LAV[1], ad.A[1]));
-  const double M2 = fma(pD, DA_DEL[2], fma(pL, DA_LAV[2], ad.A[2]));
-  const double r0 = fma(-pD, DXE_DEL[0], fma(-pL, DXE_LAV[0], c.xCr - P.xe_g[0]));
-  const double r1 = fma(-pD, DXE_DEL[1], fma(-pL, DXE_LAV[1], c.xNb - P.xe_g[1]));
-  const double det = fma(M0, M2, -(M1 * M1));
-  const double inv = sizeof(T) == sizeof(float) ? recip1(det) : recip(det);
-  v.mu0 = fma(M2, r0, -(M1 * r1)) * inv;
-  v.mu1 = fma(M0, r1, -(M1 * r0)) * inv;
+  solve(coefficients<T>(ad, v.pd, v.pl), c, v);
 }
 
 __device__ __forceinline__ Point shift_left(const Point& a) {
@@ -277,6 +293,10 @@ __device__ __forceinline__ void nucleate_cell(const NucParams& N, uint32_t cell,
 // folded symmetric five-point one (m[1] = m[7] = 1, m[3] = m[5]; the factor
 // the caller's mask had at m[1] is in q and k), and a Laplacian is
 // (S + N) + m[3] (W + E) + m[4] C.
+__device__ __forceinline__ double five_point(const double* m, double s, double w, double c,
+                                             double e, double n) {
+  return fma(m[4], c, fma(m[3], w + e, s + n));
+}
 template <bool NINE>
 __device__ __forceinline__ void laplacians(const double* m, const Point& S, const Point& W,
                                            const Point& C, const Point& E, const Point& Nn,
@@ -305,8 +325,7 @@ __device__ __forceinline__ void laplacians(const double* m, const Point& S, cons
       v = fma(m[7], n[f], v);
       v = fma(m[8], ne[f], v);
     } else {
-      v = fma(m[3], w[f] + e[f], s[f] + n[f]);
-      v = fma(m[4], c[f], v);
+      v = five_point(m, s[f], w[f], c[f], e[f], n[f]);
     }
     lap[f] = v;
   }
@@ -325,11 +344,16 @@ __device__ __forceinline__ void laplacians(const double* m, const Point& S, cons
 // state per level, the quadratic form is evaluated in two brackets with no
 // squares, and u (G u + w (2 phi - 1)) and c phi phi_o^2 are folded into
 // FMAs: 33 operations after the Laplacians, 41 with the terms written out.
+__device__ __forceinline__ void update_compositions(const StepParams& P, const Addends& ad,
+                                                    const double lap_mu[2], const Centre& cc,
+                                                    double& nCr, double& nNb) {
+  nCr = cc.xCr + fma(P.qCr[0], lap_mu[0], fma(P.qCr[1], lap_mu[1], ad.qs[0]));
+  nNb = cc.xNb + fma(P.qNb[0], lap_mu[0], fma(P.qNb[1], lap_mu[1], ad.qs[1]));
+}
 __device__ __forceinline__ void update_cell(const StepParams& P, const Addends& ad,
                                             const double lap[4], const Point& cur, const Centre& cc, double& nCr, double& nNb,
                                             double& npd, double& npl) {
-  nCr = cc.xCr + fma(P.qCr[0], lap[2], fma(P.qCr[1], lap[3], ad.qs[0]));
-  nNb = cc.xNb + fma(P.qNb[0], lap[2], fma(P.qNb[1], lap[3], ad.qs[1]));
+  update_compositions(P, ad, lap + 2, cc, nCr, nNb);
   const double fd = cur.pd, fl = cur.pl;
   const double Gd = fma(cur.mu0, fma(P.g[0][0], cur.mu0, fma(P.g[0][1], cur.mu1, ad.g3[0])),
                         cur.mu1 * fma(P.g[0][2], cur.mu1, ad.g4[0]));
@@ -422,9 +446,9 @@ __device__ __forceinline__ void march(
   {
     Raw<T> r;
     load(r, y0 - 1);
-    derive<T>(P, ad, r, win[2], cen[2]);
+    derive<T>(ad, r, win[2], cen[2]);
     load(r, y0);
-    derive<T>(P, ad, r, win[0], cen[0]);
+    derive<T>(ad, r, win[0], cen[0]);
   }
 #pragma unroll
   for (int j = 0; j < DEPTH; j++) load(ring[j], min(y0 + 1 + j, y1));
@@ -443,7 +467,7 @@ __device__ __forceinline__ void march(
       if (y >= y1) return;
       const int ps = (k + 2) % 3, cs = k % 3, ns = (k + 1) % 3;
       const int rs = k % DEPTH;
-      derive<T>(P, ad, ring[rs], win[ns], cen[ns]);
+      derive<T>(ad, ring[rs], win[ns], cen[ns]);
       load(ring[rs], min(y + 1 + DEPTH, y1));
 
       Point W, E;
@@ -531,14 +555,48 @@ __device__ __forceinline__ void march(
 // So K steps here give the same result as K one-step launches.  Symmetric
 // five-point masks, no nucleation (the caller runs nucleation steps one at a
 // time).
-template <typename T, int BC, int K, int DEPTH, int SW, bool LW>
+//
+// Most of a domain is matrix, away from any interface, and the march is bound
+// by the FP64 operations it issues (and the power they take), so an iteration
+// runs in one of three modes, chosen by the old rows it depends on: the 2K+1
+// newest, over the wave's 64 columns.
+//  - MATRIX: every |phi| is below PHI_MATRIX.  No level's |phi| can then reach
+//    TINY, so p - 1/2 is exactly -1/2 (p_less_half) and M, 1/det M and r - x
+//    are the same for all cells of all levels: computed once per wave, by the
+//    instructions a cell's own would be.  A solve is 8 operations, not 39.
+//  - QUIET: besides, every phi is +0.  The phase updates then give +0 by their
+//    own arithmetic, so only the compositions are updated and only the
+//    potentials exchanged.
+//  - DENSE: the general case, at the cost of the test (seven operations per
+//    row of some 430).
+// Every mode gives the bits of DENSE: StepParams::matrix_ok says (from bounds
+// on the coefficients) that a step multiplies |phi| < TINY by 16 at most, that
+// compositions below X_MATRIX keep every product finite (so 0 * G is 0), and
+// the test fails on NaN and infinity.
+enum Mode { DENSE, MATRIX, QUIET };
+
+template <typename T>
+__device__ __forceinline__ bool matrix_row(const Raw<T>& r) {
+  return __all(fabs((double)r.pd) < PHI_MATRIX && fabs((double)r.pl) < PHI_MATRIX &&
+               fabs((double)r.cr) < X_MATRIX && fabs((double)r.nb) < X_MATRIX);
+}
+__device__ __forceinline__ int set_bits(float v) { return __float_as_int(v); }
+__device__ __forceinline__ int set_bits(double v) { return __double2loint(v) | __double2hiint(v); }
+
+template <typename T, int BC, int K, int DEPTH, int SW, bool LW, bool MODES>
 __device__ __forceinline__ void marchk_impl(
     const T* __restrict__ iCr, const T* __restrict__ iNb, const T* __restrict__ ipd,
     const T* __restrict__ ipl, T* __restrict__ oCr, T* __restrict__ oNb, T* __restrict__ opd,
     T* __restrict__ opl, int Nx, int Ny, int pitch, int strip, int chunk, int rows,
     const StepParams& P, LdsPtr lw) {
   static_assert(K >= 2 && K <= 4, "two to four steps per pass");
-  static_assert(UNROLL % DEPTH == 0, "ring depth must divide the unroll factor");
+  // window rows in registers.  Two live rows suffice with the rows behind in
+  // LDS; the plain march still rotates three names over six rows, which the
+  // register allocator handles best, while the march with modes, three times
+  // the code per row, takes the shortest unrolling.
+  constexpr int SLOTS = LW && MODES ? 2 : 3;
+  constexpr int UNROLL = LW && MODES ? (DEPTH % 2 ? 2 * DEPTH : DEPTH) : pf::UNROLL;
+  static_assert(UNROLL % DEPTH == 0 && UNROLL % SLOTS == 0, "ring and window rotate by unrolling");
   // SW output columns per strip (64 - 2K, or fewer where the strips are laid
   // out for a deeper march); lanes K .. K+SW-1 store
   static_assert(SW >= 1 && SW <= WAVE - 2 * K, "strip width");
@@ -557,15 +615,24 @@ __device__ __forceinline__ void marchk_impl(
   const uint32_t in_lane = (uint32_t)px * (uint32_t)sizeof(T);
   const uint32_t out_lane_b = (uint32_t)(1 + gx) * (uint32_t)sizeof(T);
   const size_t row_b = (size_t)pitch * sizeof(T);
-  auto load = [&](Raw<T>& r, int y) {
-    load_row(r, iCr, iNb, ipd, ipl, (size_t)(1 + bc_map<BC>(y, Ny)) * row_b, in_lane);
+  auto row_offset = [&](int y) { return (size_t)(1 + bc_map<BC>(y, Ny)) * row_b; };
+  auto load = [&](Raw<T>& r, size_t offset) {
+    load_row(r, iCr, iNb, ipd, ipl, offset, in_lane);
   };
   const double* m = P.m;
   const Addends ad = addends(P);
+  int matrix_rows = 0, quiet_rows = 0;  // old rows of each kind, up to the newest
+  auto inspect = [&](const Raw<T>& r) {
+    if constexpr (!MODES) return;
+    const bool mr = P.matrix_ok && matrix_row(r);
+    const bool qr = mr && __all((set_bits(r.pd) | set_bits(r.pl)) == 0);
+    matrix_rows = mr ? matrix_rows + 1 : 0;
+    quiet_rows = qr ? quiet_rows + 1 : 0;
+  };
 
   // windows: level l (0 = old fields) row of iteration t in slot t % 3
-  Point win[K][3];
-  Centre cen[K][3];
+  Point win[K][SLOTS];
+  Centre cen[K][SLOTS];
   Raw<T> ring[DEPTH];
 
   // LDS copy of the row of level l that is behind at the next iteration
@@ -587,31 +654,47 @@ __device__ __forceinline__ void marchk_impl(
     }
   };
 
-  // One step at the centre of level `lv`'s window (slots behind / centre /
-  // ahead): the next level's values, rounded to storage, derived into `v`, `c`.
-  auto level_up = [&](const Point& Sth, const Point& C, const Centre& cc, const Point& Nth,
-                      Point& v, Centre& c) {
-    const Point W = shift_left(C), E = shift_right(C);
-    double lap[4];
-    laplacians<false>(m, Sth, W, C, E, Nth, Sth, Sth, Nth, Nth, lap);
-    double n0, n1, n2, n3;
-    update_cell(P, ad, lap, C, cc, n0, n1, n2, n3);
-    Raw<T> r;
-    r.cr = (T)n0;
-    r.nb = (T)n1;
-    r.pd = (T)n2;
-    r.pl = (T)n3;
-    derive<T>(P, ad, r, v, c);
+  // a row's values as stored -> its window entry
+  Coef matrix;
+  auto enter = [&](auto mode, const Raw<T>& r, Point& v, Centre& c) {
+    v.pd = mode.value == QUIET ? 0.0 : (double)r.pd;
+    v.pl = mode.value == QUIET ? 0.0 : (double)r.pl;
+    c.xCr = (double)r.cr;
+    c.xNb = (double)r.nb;
+    if constexpr (mode.value == DENSE)
+      solve(coefficients<T>(ad, v.pd, v.pl), c, v);
+    else
+      solve(matrix, c, v);
+  };
+  // the values one step after the centre row of level l's window (slots
+  // behind / centre / ahead)
+  auto advance = [&](auto mode, int l, int sa, int sc, int sb, double n[4]) {
+    const Point S = behind(l, sb);
+    const Point& C = win[l][sc];
+    const Point& N = win[l][sa];
+    if constexpr (mode.value == QUIET) {
+      const double lap[2] = {
+          five_point(m, S.mu0, from_left(C.mu0), C.mu0, from_right(C.mu0), N.mu0),
+          five_point(m, S.mu1, from_left(C.mu1), C.mu1, from_right(C.mu1), N.mu1)};
+      update_compositions(P, ad, lap, cen[l][sc], n[0], n[1]);
+      n[2] = n[3] = 0.0;
+    } else {
+      const Point W = shift_left(C), E = shift_right(C);
+      double lap[4];
+      laplacians<false>(m, S, W, C, E, N, S, S, N, N, lap);
+      update_cell(P, ad, lap, C, cen[l][sc], n[0], n[1], n[2], n[3]);
+    }
   };
 
   // Levels 1..K-1 at iteration t (slots are compile-time in both callers):
   // level l computes row y0-K+t-l.
-  auto middle_levels = [&](int sa, int sc, int sb, int lmax_active) {
+  auto middle_levels = [&](auto mode, int sa, int sc, int sb, int lmax_active) {
 #pragma unroll
     for (int l = 1; l < K; l++) {
       if (l > lmax_active) break;
-      level_up(behind(l - 1, sb), win[l - 1][sc], cen[l - 1][sc], win[l - 1][sa], win[l][sa],
-               cen[l][sa]);
+      double n[4];
+      advance(mode, l - 1, sa, sc, sb, n);
+      enter(mode, Raw<T>{(T)n[0], (T)n[1], (T)n[2], (T)n[3]}, win[l][sa], cen[l][sa]);
     }
   };
   // end of iteration t: the centre rows of the levels active before it to
@@ -626,21 +709,29 @@ __device__ __forceinline__ void marchk_impl(
     }
   };
 
+  if constexpr (MODES) matrix = coefficients<T>(ad, 0.0, 0.0);
+
   // ---- prologue: iterations t = 0 .. 2K-1 (level K not yet active).  Every
   // row the prologue reads, and the ring, is requested before the first is
   // used, so a wave waits for one memory latency at its start, not 2K.
   {
     Raw<T> pro[2 * K];
 #pragma unroll
-    for (int t = 0; t < 2 * K; t++) load(pro[t], y0 - K + t);
+    for (int t = 0; t < 2 * K; t++) load(pro[t], row_offset(y0 - K + t));
 #pragma unroll
-    for (int j = 0; j < DEPTH; j++) load(ring[j], min(y0 + K + j, y_last));
+    for (int j = 0; j < DEPTH; j++) load(ring[j], row_offset(min(y0 + K + j, y_last)));
 #pragma unroll
     for (int t = 0; t < 2 * K; t++) {
-      const int sa = t % 3, sc = (t + 2) % 3, sb = (t + 1) % 3;
-      derive<T>(P, ad, pro[t], win[0][sa], cen[0][sa]);
-      // level l is active from iteration 2l on
-      middle_levels(sa, sc, sb, t / 2);
+      const int sa = t % SLOTS, sc = (t + SLOTS - 1) % SLOTS, sb = (t + 1) % SLOTS;
+      inspect(pro[t]);
+      auto iteration = [&](auto mode) {
+        enter(mode, pro[t], win[0][sa], cen[0][sa]);
+        middle_levels(mode, sa, sc, sb, t / 2);
+      };
+      if (MODES && matrix_rows > t)
+        iteration(std::integral_constant<Mode, MATRIX>());
+      else
+        iteration(std::integral_constant<Mode, DENSE>());
       put_rows(sc, (t + 1) / 2);
     }
   }
@@ -651,36 +742,43 @@ __device__ __forceinline__ void marchk_impl(
     for (int k = 0; k < UNROLL; k++) {
       if (ib + k >= nrows) return;
       const int y = y0 + ib + k;
-      const int sa = (2 * K + k) % 3, sc = (2 * K + k + 2) % 3, sb = (2 * K + k + 1) % 3;
+      const int sa = (2 * K + k) % SLOTS, sc = (2 * K + k + SLOTS - 1) % SLOTS,
+                sb = (2 * K + k + 1) % SLOTS;
       const int rs = k % DEPTH;
-      derive<T>(P, ad, ring[rs], win[0][sa], cen[0][sa]);  // old row y + K
-      load(ring[rs], min(y + K + DEPTH, y_last));
-      middle_levels(sa, sc, sb, K - 1);
-      // level K: row y from level K-1's rows y-1 (behind), y, y+1 (ahead)
-      const Point Sth = behind(K - 1, sb);
-      const Point& C = win[K - 1][sc];
-      const Point& Nth = win[K - 1][sa];
-      const Point W = shift_left(C), E = shift_right(C);
-      double lap[4];
-      laplacians<false>(m, Sth, W, C, E, Nth, Sth, Sth, Nth, Nth, lap);
-      double nCr, nNb, npd, npl;
-      update_cell(P, ad, lap, C, cen[K - 1][sc], nCr, nNb, npd, npl);
+      double n[4];
+      inspect(ring[rs]);
+      auto iteration = [&](auto mode) {
+        enter(mode, ring[rs], win[0][sa], cen[0][sa]);  // old row y + K
+        load(ring[rs], row_offset(min(y + K + DEPTH, y_last)));
+        middle_levels(mode, sa, sc, sb, K - 1);
+        // level K: row y
+        advance(mode, K - 1, sa, sc, sb, n);
+      };
+      if (MODES && quiet_rows > 2 * K)
+        iteration(std::integral_constant<Mode, QUIET>());
+      else if (MODES && matrix_rows > 2 * K)
+        iteration(std::integral_constant<Mode, MATRIX>());
+      else
+        iteration(std::integral_constant<Mode, DENSE>());
       if (out_lane) {
-        store_row(oCr, oNb, opd, opl, (size_t)(1 + y) * row_b, out_lane_b, nCr, nNb, npd, npl);
-        store_ghost_images<T, BC>(oCr, oNb, opd, opl, gx, y, Nx, Ny, pitch, nCr, nNb, npd, npl);
+        store_row(oCr, oNb, opd, opl, (size_t)(1 + y) * row_b, out_lane_b, n[0], n[1], n[2],
+                  n[3]);
+        store_ghost_images<T, BC>(oCr, oNb, opd, opl, gx, y, Nx, Ny, pitch, n[0], n[1], n[2],
+                                  n[3]);
       }
       put_rows(sc, K);
     }
   }
 }
 
-template <typename T, int BC, int K, int DEPTH, int SW = WAVE - 2 * K, bool LW = false>
+template <typename T, int BC, int K, int DEPTH, int SW = WAVE - 2 * K, bool LW = false,
+          bool MODES = false>
 __device__ __forceinline__ void marchk(
     const T* __restrict__ iCr, const T* __restrict__ iNb, const T* __restrict__ ipd,
     const T* __restrict__ ipl, T* __restrict__ oCr, T* __restrict__ oNb, T* __restrict__ opd,
     T* __restrict__ opl, int Nx, int Ny, int pitch, int strip, int chunk, int rows,
     const StepParams& P, LdsPtr lw = nullptr) {
-  marchk_impl<T, BC, K, DEPTH, SW, LW>(iCr, iNb, ipd, ipl, oCr, oNb, opd, opl, Nx, Ny, pitch,
+  marchk_impl<T, BC, K, DEPTH, SW, LW, MODES>(iCr, iNb, ipd, ipl, oCr, oNb, opd, opl, Nx, Ny, pitch,
                                        strip, chunk, rows, P, lw);
 }
 

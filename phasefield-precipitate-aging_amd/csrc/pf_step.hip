@@ -103,7 +103,7 @@ hipError_t launch_step(int nx, int ny, int bc, const StepParams& P, const T* iCr
 
 // ---- K steps per launch (marchk, K = 2, 3 or 4) ----
 
-template <typename T, int BC, int K, int DEPTH>
+template <typename T, int BC, int K, int DEPTH, bool MODES>
 __global__ __launch_bounds__(WAVE * WPB) void stepk_kernel(
     const T* __restrict__ iCr, const T* __restrict__ iNb, const T* __restrict__ ipd,
     const T* __restrict__ ipl, T* __restrict__ oCr, T* __restrict__ oNb, T* __restrict__ opd,
@@ -114,8 +114,8 @@ __global__ __launch_bounds__(WAVE * WPB) void stepk_kernel(
   const int b = (remap ? xcd_remap(blockIdx.x, nblocks) : (int)blockIdx.x) * WPB +
                 __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));  // wave-uniform
   if (b >= nwaves) return;
-  marchk<T, BC, K, DEPTH>(iCr, iNb, ipd, ipl, oCr, oNb, opd, opl, Nx, Ny, pitch, b % strips,
-                          b / strips, rows, P);
+  marchk<T, BC, K, DEPTH, WAVE - 2 * K, false, MODES>(iCr, iNb, ipd, ipl, oCr, oNb, opd, opl, Nx,
+                                                      Ny, pitch, b % strips, b / strips, rows, P);
 }
 
 // Four steps: the rows behind of the four levels' windows live in LDS (8 KiB
@@ -125,7 +125,7 @@ __global__ __launch_bounds__(WAVE * WPB) void stepk_kernel(
 // on a domain full of particles (380 us before the sums of update_cell were
 // nested and its constant addends kept in vector registers), 75% of it VALU
 // issue.
-template <typename T, int BC, int DEPTH>
+template <typename T, int BC, int DEPTH, bool MODES>
 __global__ __launch_bounds__(WAVE * WPB) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void step4_kernel(const T* __restrict__ iCr, const T* __restrict__ iNb,
                   const T* __restrict__ ipd, const T* __restrict__ ipl, T* __restrict__ oCr,
@@ -139,9 +139,9 @@ void step4_kernel(const T* __restrict__ iCr, const T* __restrict__ iNb,
   const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));  // wave-uniform
   const int b = (remap ? xcd_remap(blockIdx.x, nblocks) : (int)blockIdx.x) * WPB + w;
   if (b >= nwaves) return;
-  marchk<T, BC, K, DEPTH, WAVE - 2 * K, true>(iCr, iNb, ipd, ipl, oCr, oNb, opd, opl, Nx, Ny,
-                                              pitch, b % strips, b / strips, rows, P,
-                                              (LdsPtr)win_lds + w * PER_WAVE);
+  marchk<T, BC, K, DEPTH, WAVE - 2 * K, true, MODES>(iCr, iNb, ipd, ipl, oCr, oNb, opd, opl, Nx,
+                                                     Ny, pitch, b % strips, b / strips, rows, P,
+                                                     (LdsPtr)win_lds + w * PER_WAVE);
 }
 
 // Chunk height of the four-step kernel from a model of its launch on
@@ -171,6 +171,17 @@ static int rows4_model(int strips, int Ny) {
   return best;
 }
 
+// Chunks of this height and more run the march with modes (matrix and quiet
+// rows apart, pf_march.h).  Its 2K+1 dense rows at a chunk's start and three
+// times the code do not pay on short chunks (17 rows, 1400 x 1100 FP32: 39.5
+// against 36.7 us per four-step launch; 2 rows, 256^2: 10.5 against 8.8).
+// From here on, us per launch without / with modes:
+//   FP64 4096^2, 75 rows, four steps: no precipitate 300 / 265, one particle's
+//   tail over the domain 314 / 282, particles everywhere 324 / 328;
+//   FP64 2048^2, 38 rows: 80.0 / 65.6, 86.5 / 88.3 with particles everywhere;
+//   FP32 8192^2, 48 rows, three steps: 790 / 567, 802 / 818.
+constexpr int MODE_ROWS = 32;
+
 int default_rows_k(int k, int nx, int ny, int storage_bytes) {
   // The intermediate levels recompute (K-1)K rows per chunk in all, so chunks
   // are longer than the one-step kernel's while the grid still fills the chip.
@@ -198,14 +209,23 @@ static hipError_t launch_stepk_t(int nx, int ny, const StepParams& P, const T* i
   const int strips = (Nx + sw - 1) / sw;
   const int chunks = (Ny + rows - 1) / rows;
   const int blocks = (strips * chunks + WPB - 1) / WPB;
-  if constexpr (K == 4)
-    hipLaunchKernelGGL((step4_kernel<T, BC, DEPTH>), dim3(blocks), dim3(WAVE * WPB), 0, st, iCr,
-                       iNb, ipd, ipl, oCr, oNb, opd, opl, Nx, Ny, nx, strips, chunks, rows, remap,
-                       P);
-  else
-    hipLaunchKernelGGL((stepk_kernel<T, BC, K, DEPTH>), dim3(blocks), dim3(WAVE * WPB), 0, st,
-                       iCr, iNb, ipd, ipl, oCr, oNb, opd, opl, Nx, Ny, nx, strips, chunks, rows,
-                       remap, P);
+#define PF_LAUNCH_MARCH(KERNEL)                                                                 \
+  hipLaunchKernelGGL(KERNEL, dim3(blocks), dim3(WAVE * WPB), 0, st, iCr, iNb, ipd, ipl, oCr,    \
+                     oNb, opd, opl, Nx, Ny, nx, strips, chunks, rows, remap, P)
+  if constexpr (K == 4) {
+    if (rows >= MODE_ROWS)
+      PF_LAUNCH_MARCH((step4_kernel<T, BC, 4, true>));
+    else
+      PF_LAUNCH_MARCH((step4_kernel<T, BC, DEPTH, false>));
+  } else if constexpr (K == 3 && sizeof(T) == sizeof(float)) {
+    if (rows >= MODE_ROWS)
+      PF_LAUNCH_MARCH((stepk_kernel<T, BC, K, 3, true>));
+    else
+      PF_LAUNCH_MARCH((stepk_kernel<T, BC, K, DEPTH, false>));
+  } else {
+    PF_LAUNCH_MARCH((stepk_kernel<T, BC, K, DEPTH, false>));
+  }
+#undef PF_LAUNCH_MARCH
   return hipGetLastError();
 }
 
