@@ -28,8 +28,8 @@ hipError_t scratch_alloc(Scratch& s) {
   if (e != hipSuccess) return e;
   e = hipMalloc((void**)&s.events, (size_t)s.event_capacity * sizeof(Event));
   if (e != hipSuccess) return e;
-  // per-block partials of up to 5 compensated sums, then 8 doubles of final sums
-  e = hipMalloc((void**)&s.partials, ((size_t)REDUCE_BLOCKS * 10 + 8) * sizeof(double));
+  // per-block partials of up to 5 compensated sums
+  e = hipMalloc((void**)&s.partials, (size_t)REDUCE_BLOCKS * 10 * sizeof(double));
   return e;
 }
 void scratch_free(Scratch& s) {
@@ -293,17 +293,38 @@ __device__ __forceinline__ void kmerge(Kahan& a, const Kahan& b) {
   a.c += b.c;
 }
 
+// Position of a thread's next interior cell in a grid-stride walk over rows of
+// Nx cells: a division at the start and none per cell.  `block` is the block's
+// place in the walk.
+struct Walk {
+  int x, y, dx, dy, Nx;
+  __device__ __forceinline__ Walk(int block, int Nx_) : Nx(Nx_) {
+    const unsigned first = block * 256u + threadIdx.x, stride = gridDim.x * 256u;
+    y = (int)(first / (unsigned)Nx);
+    x = (int)(first - (unsigned)y * (unsigned)Nx);
+    dy = (int)(stride / (unsigned)Nx);
+    dx = (int)(stride - (unsigned)dy * (unsigned)Nx);
+  }
+  __device__ __forceinline__ void next() {
+    x += dx;
+    y += dy;
+    if (x >= Nx) {
+      x -= Nx;
+      y++;
+    }
+  }
+};
+
 template <typename T>
 __global__ __launch_bounds__(256) void summarize_partial_kernel(const T* __restrict__ xCr,
                                                                 const T* __restrict__ xNb,
                                                                 const T* __restrict__ pd,
                                                                 const T* __restrict__ pl, int nx,
                                                                 int ny, double* partials) {
-  const long Nx = nx - 2, Ny = ny - 2, N = Nx * Ny;
+  const int Ny = ny - 2;
   Kahan acc[5] = {};
-  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < N; i += (long)gridDim.x * 256) {
-    const long y = i / Nx, x = i - y * Nx;
-    const size_t o = (size_t)(y + 1) * nx + (x + 1);
+  for (Walk w(blockIdx.x, nx - 2); w.y < Ny; w.next()) {
+    const size_t o = (size_t)(w.y + 1) * nx + (w.x + 1);
     const double d = p((double)pd[o]), l = p((double)pl[o]);
     kadd(acc[0], (double)xCr[o]);
     kadd(acc[1], (double)xNb[o]);
@@ -327,26 +348,39 @@ __global__ __launch_bounds__(256) void summarize_partial_kernel(const T* __restr
 }
 
 // Final pass over the per-block partials of `nq` quantities (stride 2*nq
-// doubles per block): block k merges quantity k, 64 threads over a fixed
-// partition, then a fixed tree.  out[k] = sum * scale (+ add0 / add1 for
-// quantities 0 / 1).
+// doubles per block): a wave merges quantity k, its 64 lanes over a fixed
+// partition, then a fixed tree.  A lane requests its partials, at most
+// REDUCE_BLOCKS / 64, before it merges the first.  Returns the sum on every
+// lane, so the energy's two sums and their total take one launch.
+__device__ __forceinline__ double merge_partials(const double* partials, int nblocks, int nq,
+                                                 int k) {
+  const int t = threadIdx.x & 63;
+  constexpr int MOST = REDUCE_BLOCKS / 64;
+  Kahan v[MOST];
+#pragma unroll
+  for (int j = 0; j < MOST; j++) {
+    const int b = min(t + 64 * j, nblocks - 1);
+    v[j] = Kahan{partials[(size_t)b * 2 * nq + 2 * k], partials[(size_t)b * 2 * nq + 2 * k + 1]};
+  }
+  Kahan a{0.0, 0.0};
+#pragma unroll
+  for (int j = 0; j < MOST; j++)
+    if (t + 64 * j < nblocks) kmerge(a, v[j]);
+#pragma unroll
+  for (int w = 32; w > 0; w >>= 1) {
+    const Kahan o{__shfl_down(a.s, w), __shfl_down(a.c, w)};
+    if (t < w) kmerge(a, o);
+  }
+  return __shfl(a.s + a.c, 0);
+}
+
+// out[k] = sum * scale (+ add0 / add1 for quantities 0 / 1), block k
 __global__ __launch_bounds__(64) void reduce_final_kernel(const double* partials, int nblocks,
                                                           int nq, double scale, double* out,
                                                           double add0, double add1) {
-  const int k = blockIdx.x, t = threadIdx.x;
-  Kahan a{0.0, 0.0};
-  for (int b = t; b < nblocks; b += 64) {
-    Kahan v{partials[(size_t)b * 2 * nq + 2 * k], partials[(size_t)b * 2 * nq + 2 * k + 1]};
-    kmerge(a, v);
-  }
-  __shared__ Kahan sh[64];
-  sh[t] = a;
-  __syncthreads();
-  for (int w = 32; w > 0; w >>= 1) {
-    if (t < w) kmerge(sh[t], sh[t + w]);
-    __syncthreads();
-  }
-  if (t == 0) out[k] = (sh[0].s + sh[0].c) * scale + (k == 0 ? add0 : (k == 1 ? add1 : 0.0));
+  const int k = blockIdx.x;
+  const double sum = merge_partials(partials, nblocks, nq, k);
+  if (threadIdx.x == 0) out[k] = sum * scale + (k == 0 ? add0 : (k == 1 ? add1 : 0.0));
 }
 
 // The mean compositions are the offset plus the mean of the stored values.
@@ -389,10 +423,14 @@ __global__ __launch_bounds__(256) void energy_partial_kernel(
     const T* __restrict__ pl, int nx, int ny, EnergyParams E, double* __restrict__ chem_out,
     double* __restrict__ grad_out, double* partials) {
   const int Nx = nx - 2, Ny = ny - 2;
-  const long N = (long)Nx * Ny;
+  // a contiguous band of cells per XCD in each stride of the grid, so that the
+  // rows above and below mostly come from its own L2 (bound by the traffic of
+  // the neighbour rows: 3000^2 FP64 84 -> 78 us)
+  const int block = xcd_remap(blockIdx.x, gridDim.x);
   Kahan acc[2] = {};
-  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < N; i += (long)gridDim.x * 256) {
-    const int y = (int)(i / Nx), x = (int)(i - (long)y * Nx);
+  const double rx = 1.0 / (2.0 * E.dx), ry = 1.0 / (2.0 * E.dy);
+  for (Walk w(block, Nx); w.y < Ny; w.next()) {
+    const int x = w.x, y = w.y;
     const size_t o = (size_t)(y + 1) * nx + (x + 1);
     const double cr = (double)xCr[o] + E.xoff[0], nb = (double)xNb[o] + E.xoff[1];
     const double fd = (double)pd[o], fl = (double)pl[o];
@@ -413,8 +451,8 @@ __global__ __launch_bounds__(256) void energy_partial_kernel(
     double ge = 0.0;
 #pragma unroll
     for (int k = 0; k < 2; k++) {
-      const double gx = ((double)phi[k][xh] - (double)phi[k][xl]) / (2.0 * E.dx);
-      const double gy = ((double)phi[k][yh] - (double)phi[k][yl]) / (2.0 * E.dy);
+      const double gx = ((double)phi[k][xh] - (double)phi[k][xl]) * rx;
+      const double gy = ((double)phi[k][yh] - (double)phi[k][yl]) * ry;
       ge += E.kappa[k] * (gx * gx + gy * gy);
     }
     const double c = g * E.dV, gg = ge * E.dV;
@@ -433,16 +471,23 @@ __global__ __launch_bounds__(256) void energy_partial_kernel(
   }
   if (threadIdx.x == 0)
     for (int k = 0; k < 2; k++) {
-      partials[(size_t)blockIdx.x * 4 + 2 * k] = sh[k][0].s;
-      partials[(size_t)blockIdx.x * 4 + 2 * k + 1] = sh[k][0].c;
+      partials[(size_t)block * 4 + 2 * k] = sh[k][0].s;
+      partials[(size_t)block * 4 + 2 * k + 1] = sh[k][0].c;
     }
 }
 
-__global__ void energy_total_kernel(const double* sums, double* out3) {
+// out3 = {chemical + gradient, chemical, gradient}, one wave per sum
+__global__ __launch_bounds__(128) void energy_final_kernel(const double* partials, int nblocks,
+                                                           double* out3) {
+  __shared__ double sums[2];
+  const int k = threadIdx.x >> 6;
+  const double sum = merge_partials(partials, nblocks, 2, k);
+  if ((threadIdx.x & 63) == 0) sums[k] = sum;
+  __syncthreads();
   if (threadIdx.x == 0) {
+    out3[0] = sums[0] + sums[1];
     out3[1] = sums[0];
     out3[2] = sums[1];
-    out3[0] = sums[0] + sums[1];
   }
 }
 
@@ -462,12 +507,7 @@ hipError_t launch_energy(int nx, int ny, int bc, const EnergyParams& E, const T*
                        pd, pl, nx, ny, E, chem, grad, S.partials);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  // the two sums land in out3[1..2] via a scratch slot after the partials
-  double* sums = S.partials + (size_t)REDUCE_BLOCKS * 10;
-  hipLaunchKernelGGL(reduce_final_kernel, dim3(2), dim3(64), 0, st, S.partials, blocks, 2, 1.0,
-                     sums, 0.0, 0.0);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  hipLaunchKernelGGL(energy_total_kernel, dim3(1), dim3(64), 0, st, sums, out3);
+  hipLaunchKernelGGL(energy_final_kernel, dim3(1), dim3(128), 0, st, S.partials, blocks, out3);
   return hipGetLastError();
 }
 template hipError_t launch_energy<double>(int, int, int, const EnergyParams&, const double*,

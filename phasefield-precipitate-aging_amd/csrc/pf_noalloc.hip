@@ -2,7 +2,7 @@
 // pf_summarize_f64 for callers that cannot allocate device memory (code under
 // HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
 // It needs no context: the reduction partials live in a file-scope device
-// array, `scratch`, of fixed size (REDUCE_BLOCKS * 10 + 8 doubles, 80 KiB),
+// array, `scratch`, of fixed size (REDUCE_BLOCKS * 10 doubles, 80 KiB),
 // which every GPU the library runs on holds until the process ends.  The call
 // allocates nothing and calls no allocating routine.
 //
@@ -22,7 +22,7 @@
 
 namespace pf {
 
-constexpr size_t NOALLOC_SCRATCH_DOUBLES = (size_t)REDUCE_BLOCKS * 10 + 8;
+constexpr size_t NOALLOC_SCRATCH_DOUBLES = (size_t)REDUCE_BLOCKS * 10;
 
 static __device__ __align__(256) double scratch[NOALLOC_SCRATCH_DOUBLES];
 

@@ -260,17 +260,15 @@ class Simulation:
         return out
 
     def summarize(self):
-        # allocated and cleared on the simulation's stream, in order with the
-        # reduction that writes it (a stream of its own need not wait for the
-        # current one)
+        # allocated, written by the reduction and read back on the simulation's
+        # stream (a stream of its own need not wait for the current one)
         with torch.cuda.stream(self.stream):
-            out = torch.zeros(5, dtype=torch.float64, device="cuda")
-        a = self.a
-        check(self._summ(self.ctx, self.nx, self.ny, _ptr(a[0]), _ptr(a[1]), _ptr(a[2]),
-                         _ptr(a[3]), _ptr(out), ctypes.c_void_p(self.stream.cuda_stream)),
-              "pf_summarize")
-        self.stream.synchronize()
-        return out.cpu().tolist()
+            out = torch.empty(5, dtype=torch.float64, device="cuda")
+            a = self.a
+            check(self._summ(self.ctx, self.nx, self.ny, _ptr(a[0]), _ptr(a[1]), _ptr(a[2]),
+                             _ptr(a[3]), _ptr(out), ctypes.c_void_p(self.stream.cuda_stream)),
+                  "pf_summarize")
+            return out.tolist()
 
     def energy(self, maps=False):
         """Free energy of the current fields (src/alloy625.cpp:865-919):
@@ -283,7 +281,7 @@ class Simulation:
         omega = (ctypes.c_double * 2)(*s.omega)
         chem = grad = None
         with torch.cuda.stream(self.stream):
-            out = torch.zeros(3, dtype=torch.float64, device="cuda")
+            out = torch.empty(3, dtype=torch.float64, device="cuda")
             if maps:
                 chem = torch.zeros(self.nx * self.ny, dtype=torch.float64, device="cuda")
                 grad = torch.zeros_like(chem)
@@ -292,8 +290,8 @@ class Simulation:
                  _ptr(a[0]), _ptr(a[1]), _ptr(a[2]), _ptr(a[3]),
                  _ptr(chem) if maps else None, _ptr(grad) if maps else None, _ptr(out),
                  ctypes.c_void_p(self.stream.cuda_stream)), "pf_energy")
-        self.stream.synchronize()
-        tot = tuple(out.cpu().tolist())
+        with torch.cuda.stream(self.stream):
+            tot = tuple(out.tolist())
         if maps:
             return tot, chem.reshape(self.ny, self.nx).cpu().numpy(), \
                 grad.reshape(self.ny, self.nx).cpu().numpy()
