@@ -144,6 +144,21 @@ int pf_step4_f32(pf_ctx* ctx, int nx, int ny, int bc, const pf_params* prm,
                  float* conc_Cr_new, float* conc_Nb_new,
                  float* phi_del_new, float* phi_lav_new, void* stream);
 
+/* `steps` steps without nucleation between two field sets a and b (four device
+ * arrays each: conc_Cr, conc_Nb, phi_del, phi_lav), a holding the current
+ * fields: the same as that many pf_step_* calls with the sets swapped after
+ * each (src/main.cpp:289-305, 318-321), issued as launches of up to
+ * steps_per_launch (1 to 4) steps.  Masks that are neither symmetric
+ * five-point nor symmetric nine-point, and grids too small for multi-step
+ * launches, run one step per launch.  *in_b (HOST) is 1 if the last step's
+ * fields are in set b, 0 if in set a; the other set is overwritten. */
+int pf_advance_f64(pf_ctx* ctx, int nx, int ny, int bc, const pf_params* prm,
+                   double* const* a, double* const* b, uint64_t steps, int steps_per_launch,
+                   int* in_b, void* stream);
+int pf_advance_f32(pf_ctx* ctx, int nx, int ny, int bc, const pf_params* prm,
+                   float* const* a, float* const* b, uint64_t steps, int steps_per_launch,
+                   int* in_b, void* stream);
+
 /* Standalone nucleation pass in place on the given fields.  Replaces
  * device_nucleation (src/discretization.cu:1179-1209). */
 int pf_nucleation_f64(pf_ctx* ctx, int nx, int ny, double* conc_Cr, double* conc_Nb,

@@ -126,7 +126,7 @@ __global__ __launch_bounds__(WAVE * WPB) void batch_step_kernel(const BatchJob* 
                                      out + 2 * pl, out + 3 * pl, J.Nx, J.Ny, J.pitch, strip,   \
                                      chunk, J.rows, J.P);                                      \
   else                                                                                       \
-    march<T, BCV, false, false, DEPTH, STRIP3>(in, in + pl, in + 2 * pl, in + 3 * pl, out,     \
+    march<T, BCV, FIVE, false, DEPTH, STRIP3>(in, in + pl, in + 2 * pl, in + 3 * pl, out,     \
                                                out + pl, out + 2 * pl, out + 3 * pl, J.Nx,    \
                                                J.Ny, J.pitch, strip, chunk, J.rows, J.P, N, S)
     if (J.bc == 0) {

@@ -137,6 +137,47 @@ int stepk_t(int k, pf_ctx* ctx, int nx, int ny, int bc, const pf_params* prm, co
   return PF_OK;
 }
 
+// `steps` plain steps from set a, alternating between the sets, up to `most`
+// per launch where the mask and the grid take multi-step launches.
+template <typename T>
+int advance_t(pf_ctx* ctx, int nx, int ny, int bc, const pf_params* prm, T* const* a,
+              T* const* b, uint64_t steps, int most, int* in_b, void* stream) {
+  if (!ctx || !prm || !a || !b || !in_b) return fail(PF_ERR_ARG, "null argument");
+  if (most < 1 || most > 4) return fail(PF_ERR_ARG, "steps per launch must be 1, 2, 3 or 4");
+  if (int r = check_grid(nx, ny)) return r;
+  if (int r = check_ptrs(a[0], a[1], a[2], a[3])) return r;
+  if (int r = check_ptrs(b[0], b[1], b[2], b[3])) return r;
+  if (bc != PF_BC_NOFLUX && bc != PF_BC_PERIODIC) return fail(PF_ERR_ARG, "unknown boundary mode");
+  if (int r = check_disjoint<T>(nx, ny, a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3])) return r;
+  // a also is written (from the second launch on): its arrays must differ
+  if (int r = check_disjoint<T>(nx, ny, b[0], b[1], b[2], b[3], a[0], a[1], a[2], a[3])) return r;
+  const pf::StepParams P = pf::make_step(prm->dt, prm->DCr, prm->DNb, prm->kappa, prm->omega,
+                                         prm->Lmob, prm->alpha, prm->mask, storage_offset<T>(ctx));
+  const bool five = pf::symmetric_five_point(prm->mask);
+  const bool nine = !five && pf::symmetric_nine_point(prm->mask);
+  if (!(five || nine) || nx < 5 || ny < 5) most = 1;
+  if (most == 4 && (nx < 6 || ny < 6)) most = 3;
+  hipStream_t st = (hipStream_t)stream;
+  int flip = 0;
+  *in_b = 0;
+  while (steps > 0) {
+    int k = steps < (uint64_t)most ? (int)steps : most;
+    if (nine && k == 3) k = 2;
+    T* const* i = flip ? b : a;
+    T* const* o = flip ? a : b;
+    const hipError_t e =
+        k == 1 ? pf::launch_step<T>(nx, ny, bc, P, i[0], i[1], i[2], i[3], o[0], o[1], o[2], o[3],
+                                    nullptr, ctx->scratch, ctx->tile, st)
+               : pf::launch_stepk<T>(k, nx, ny, bc, P, i[0], i[1], i[2], i[3], o[0], o[1], o[2],
+                                     o[3], ctx->tile, st);
+    if (e != hipSuccess) return hip_fail(e, "step kernel");
+    flip ^= 1;
+    *in_b = flip;
+    steps -= (uint64_t)k;
+  }
+  return PF_OK;
+}
+
 int set_tile_k(pf_ctx* ctx, int k, int rows, int depth) {
   if (!ctx) return fail(PF_ERR_ARG, "null context");
   if (rows < 0 || rows > 1 << 20) return fail(PF_ERR_ARG, "rows out of range");
@@ -323,6 +364,18 @@ int pf_step4_f32(pf_ctx* ctx, int nx, int ny, int bc, const pf_params* prm, cons
                  const float* b, const float* c, const float* d, float* oa, float* ob,
                  float* oc, float* od, void* stream) {
   return stepk_t<float>(4, ctx, nx, ny, bc, prm, a, b, c, d, oa, ob, oc, od, stream);
+}
+
+int pf_advance_f64(pf_ctx* ctx, int nx, int ny, int bc, const pf_params* prm, double* const* a,
+                   double* const* b, uint64_t steps, int steps_per_launch, int* in_b,
+                   void* stream) {
+  return advance_t<double>(ctx, nx, ny, bc, prm, a, b, steps, steps_per_launch, in_b, stream);
+}
+
+int pf_advance_f32(pf_ctx* ctx, int nx, int ny, int bc, const pf_params* prm, float* const* a,
+                   float* const* b, uint64_t steps, int steps_per_launch, int* in_b,
+                   void* stream) {
+  return advance_t<float>(ctx, nx, ny, bc, prm, a, b, steps, steps_per_launch, in_b, stream);
 }
 
 int pf_step_loop_f64(pf_ctx* ctx, int n, const pf_step_item* items, void* stream) {

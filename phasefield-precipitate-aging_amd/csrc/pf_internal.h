@@ -63,6 +63,12 @@ inline bool folded_five_point(const double* m) {
          m[7] == 1.0 && m[3] == m[5];
 }
 
+// Masks symmetric in x and y with corners (the reference's nine-point one).
+inline bool symmetric_nine_point(const double* m) {
+  return m[0] != 0.0 && m[0] == m[2] && m[0] == m[6] && m[0] == m[8] && m[1] == m[7] &&
+         m[3] == m[5];
+}
+
 // Nucleation pass parameters, derived on the host from the reference's
 // device_nucleation arguments (src/discretization.cu:1179-1209).
 struct NucParams {
@@ -126,8 +132,8 @@ hipError_t launch_step(int nx, int ny, int bc, const StepParams& P, const T* iCr
                        const T* ipd, const T* ipl, T* oCr, T* oNb, T* opd, T* opl,
                        const NucParams* nuc, const Scratch& S, const TileConfig& tc,
                        hipStream_t st);
-// k = 2, 3 or 4 steps per launch (folded symmetric five-point mask, no nucleation); grids
-// need Nx, Ny >= 3 (k = 4: >= 4)
+// k = 2, 3 or 4 steps per launch (folded symmetric five-point mask, or k = 2 or 4 and a
+// symmetric nine-point one; no nucleation); grids need Nx, Ny >= 3 (k = 4: >= 4)
 template <typename T>
 hipError_t launch_stepk(int k, int nx, int ny, int bc, const StepParams& P, const T* iCr,
                         const T* iNb, const T* ipd, const T* ipl, T* oCr, T* oNb, T* opd,

@@ -287,48 +287,67 @@ __device__ __forceinline__ void nucleate_cell(const NucParams& N, uint32_t cell,
   }
 }
 
-// Laplacians of the four stencil quantities with the reference's mask
+// Laplacians of the four stencil quantities with the reference's masks
 // (src/discretization.cu:589-595): rows y-1, y, y+1; columns x-1, x, x+1.
-// NINE: the general nine-term sum in mask order.  Otherwise the mask is a
-// folded symmetric five-point one (m[1] = m[7] = 1, m[3] = m[5]; the factor
-// the caller's mask had at m[1] is in q and k), and a Laplacian is
+// FIVE: a folded symmetric five-point mask (m[1] = m[7] = 1, m[3] = m[5]; the
+// factor the caller's mask had at m[1] is in q and k).  A Laplacian is
 // (S + N) + m[3] (W + E) + m[4] C.
+// NINE: a mask symmetric in x and y (the reference's nine-point one).  Its
+// west and east columns are alike, so a lane forms its column's share of its
+// neighbours' Laplacians, m[0] (S + N) + m[3] C, and only that is exchanged:
+// 7 operations and one shift each way per value, 9 and three rows' shifted
+// neighbours kept in registers for ANY.
+// Both add mirror images in the same order, which the multi-step march's
+// no-flux halo rests on.
+// ANY: the nine-term sum in mask order.
+enum Mask { FIVE, NINE, ANY };
+
 __device__ __forceinline__ double five_point(const double* m, double s, double w, double c,
                                              double e, double n) {
   return fma(m[4], c, fma(m[3], w + e, s + n));
 }
-template <bool NINE>
-__device__ __forceinline__ void laplacians(const double* m, const Point& S, const Point& W,
-                                           const Point& C, const Point& E, const Point& Nn,
-                                           const Point& SW, const Point& SE, const Point& NW,
-                                           const Point& NE, double lap[4]) {
-  const double s[4] = {S.pd, S.pl, S.mu0, S.mu1};
-  const double w[4] = {W.pd, W.pl, W.mu0, W.mu1};
-  const double c[4] = {C.pd, C.pl, C.mu0, C.mu1};
-  const double e[4] = {E.pd, E.pl, E.mu0, E.mu1};
-  const double n[4] = {Nn.pd, Nn.pl, Nn.mu0, Nn.mu1};
-#pragma unroll
-  for (int f = 0; f < 4; f++) {
-    double v;
-    if (NINE) {
-      const double sw[4] = {SW.pd, SW.pl, SW.mu0, SW.mu1};
-      const double se[4] = {SE.pd, SE.pl, SE.mu0, SE.mu1};
-      const double nw[4] = {NW.pd, NW.pl, NW.mu0, NW.mu1};
-      const double ne[4] = {NE.pd, NE.pl, NE.mu0, NE.mu1};
-      v = m[0] * sw[f];
-      v = fma(m[1], s[f], v);
-      v = fma(m[2], se[f], v);
-      v = fma(m[3], w[f], v);
-      v = fma(m[4], c[f], v);
-      v = fma(m[5], e[f], v);
-      v = fma(m[6], nw[f], v);
-      v = fma(m[7], n[f], v);
-      v = fma(m[8], ne[f], v);
-    } else {
-      v = five_point(m, s[f], w[f], c[f], e[f], n[f]);
-    }
-    lap[f] = v;
+template <Mask MASK>
+__device__ __forceinline__ double stencil(const double* m, double s, double c, double n) {
+  if constexpr (MASK == FIVE) {
+    return five_point(m, s, from_left(c), c, from_right(c), n);
+  } else {
+    const double sn = s + n, column = fma(m[0], sn, m[3] * c);
+    return (from_left(column) + from_right(column)) + fma(m[4], c, m[1] * sn);
   }
+}
+template <Mask MASK>
+__device__ __forceinline__ void laplacians(const double* m, const Point& S, const Point& C,
+                                           const Point& N, double lap[4]) {
+  lap[0] = stencil<MASK>(m, S.pd, C.pd, N.pd);
+  lap[1] = stencil<MASK>(m, S.pl, C.pl, N.pl);
+  lap[2] = stencil<MASK>(m, S.mu0, C.mu0, N.mu0);
+  lap[3] = stencil<MASK>(m, S.mu1, C.mu1, N.mu1);
+}
+__device__ __forceinline__ double nine_terms(const double* m, double sw, double s, double se,
+                                             double w, double c, double e, double nw, double n,
+                                             double ne) {
+  double v = m[0] * sw;
+  v = fma(m[1], s, v);
+  v = fma(m[2], se, v);
+  v = fma(m[3], w, v);
+  v = fma(m[4], c, v);
+  v = fma(m[5], e, v);
+  v = fma(m[6], nw, v);
+  v = fma(m[7], n, v);
+  return fma(m[8], ne, v);
+}
+// ANY: win, winW, winE hold rows y-1, y, y+1 in slots p, c, n
+__device__ __forceinline__ void laplacians_any(const double* m, const Point* win,
+                                               const Point* winW, const Point* winE, int p,
+                                               int c, int n, double lap[4]) {
+#define PF_TERMS(F)                                                                          \
+  nine_terms(m, winW[p].F, win[p].F, winE[p].F, winW[c].F, win[c].F, winE[c].F, winW[n].F,   \
+             win[n].F, winE[n].F)
+  lap[0] = PF_TERMS(pd);
+  lap[1] = PF_TERMS(pl);
+  lap[2] = PF_TERMS(mu0);
+  lap[3] = PF_TERMS(mu1);
+#undef PF_TERMS
 }
 
 // The explicit Euler update of one cell from its stencil Laplacians:
@@ -411,7 +430,7 @@ __device__ __forceinline__ void store_ghost_images(T* oCr, T* oNb, T* opd, T* op
 // step, reading the old fields and writing the new ones.  Called by a whole
 // wave; uses no barriers.  SW is the number of output columns per strip (62,
 // or 60 where the strips are laid out for the two-step march).
-template <typename T, int BC, bool NINE, bool NUC, int DEPTH, int SW = STRIP>
+template <typename T, int BC, Mask MASK, bool NUC, int DEPTH, int SW = STRIP>
 __device__ __forceinline__ void march(
     const T* __restrict__ iCr, const T* __restrict__ iNb, const T* __restrict__ ipd,
     const T* __restrict__ ipl, T* __restrict__ oCr, T* __restrict__ oNb, T* __restrict__ opd,
@@ -440,7 +459,7 @@ __device__ __forceinline__ void march(
   // window slots (row y0 + k - 1 + 3j lives in slot k % 3 pattern below)
   Point win[3];
   Centre cen[3];
-  Point winW[3], winE[3];  // DPP-shifted neighbours (nine-point masks only)
+  Point winW[3], winE[3];  // DPP-shifted neighbours (ANY only)
   Raw<T> ring[DEPTH];
 
   {
@@ -452,7 +471,7 @@ __device__ __forceinline__ void march(
   }
 #pragma unroll
   for (int j = 0; j < DEPTH; j++) load(ring[j], min(y0 + 1 + j, y1));
-  if (NINE) {
+  if (MASK == ANY) {
     winW[2] = shift_left(win[2]);
     winE[2] = shift_right(win[2]);
     winW[0] = shift_left(win[0]);
@@ -470,19 +489,14 @@ __device__ __forceinline__ void march(
       derive<T>(ad, ring[rs], win[ns], cen[ns]);
       load(ring[rs], min(y + 1 + DEPTH, y1));
 
-      Point W, E;
-      if (NINE) {
+      double lap[4];
+      if constexpr (MASK == ANY) {
         winW[ns] = shift_left(win[ns]);
         winE[ns] = shift_right(win[ns]);
-        W = winW[cs];
-        E = winE[cs];
+        laplacians_any(m, win, winW, winE, ps, cs, ns, lap);
       } else {
-        W = shift_left(win[cs]);
-        E = shift_right(win[cs]);
+        laplacians<MASK>(m, win[ps], win[cs], win[ns], lap);
       }
-      double lap[4];
-      laplacians<NINE>(m, win[ps], W, win[cs], E, win[ns], winW[ps], winE[ps], winW[ns],
-                       winE[ns], lap);
 
       double nCr, nNb, npd, npl;
       update_cell(P, ad, lap, win[cs], cen[cs], nCr, nNb, npd, npl);
@@ -553,7 +567,7 @@ __device__ __forceinline__ void march(
 //    which is the ghost copy a one-step launch makes.  So no image needs a
 //    fix-up.
 // So K steps here give the same result as K one-step launches.  Symmetric
-// five-point masks, no nucleation (the caller runs nucleation steps one at a
+// masks (FIVE, NINE), no nucleation (the caller runs nucleation steps one at a
 // time).
 //
 // Most of a domain is matrix, away from any interface, and the march is bound
@@ -583,13 +597,14 @@ __device__ __forceinline__ bool matrix_row(const Raw<T>& r) {
 __device__ __forceinline__ int set_bits(float v) { return __float_as_int(v); }
 __device__ __forceinline__ int set_bits(double v) { return __double2loint(v) | __double2hiint(v); }
 
-template <typename T, int BC, int K, int DEPTH, int SW, bool LW, bool MODES>
+template <typename T, int BC, int K, int DEPTH, int SW, bool LW, bool MODES, Mask MASK>
 __device__ __forceinline__ void marchk_impl(
     const T* __restrict__ iCr, const T* __restrict__ iNb, const T* __restrict__ ipd,
     const T* __restrict__ ipl, T* __restrict__ oCr, T* __restrict__ oNb, T* __restrict__ opd,
     T* __restrict__ opl, int Nx, int Ny, int pitch, int strip, int chunk, int rows,
     const StepParams& P, LdsPtr lw) {
   static_assert(K >= 2 && K <= 4, "two to four steps per pass");
+  static_assert(MASK == FIVE || (MASK == NINE && !MODES), "symmetric masks; modes for FIVE");
   // window rows in registers.  Two live rows suffice with the rows behind in
   // LDS; the plain march still rotates three names over six rows, which the
   // register allocator handles best, while the march with modes, three times
@@ -673,15 +688,13 @@ __device__ __forceinline__ void marchk_impl(
     const Point& C = win[l][sc];
     const Point& N = win[l][sa];
     if constexpr (mode.value == QUIET) {
-      const double lap[2] = {
-          five_point(m, S.mu0, from_left(C.mu0), C.mu0, from_right(C.mu0), N.mu0),
-          five_point(m, S.mu1, from_left(C.mu1), C.mu1, from_right(C.mu1), N.mu1)};
+      const double lap[2] = {stencil<MASK>(m, S.mu0, C.mu0, N.mu0),
+                             stencil<MASK>(m, S.mu1, C.mu1, N.mu1)};
       update_compositions(P, ad, lap, cen[l][sc], n[0], n[1]);
       n[2] = n[3] = 0.0;
     } else {
-      const Point W = shift_left(C), E = shift_right(C);
       double lap[4];
-      laplacians<false>(m, S, W, C, E, N, S, S, N, N, lap);
+      laplacians<MASK>(m, S, C, N, lap);
       update_cell(P, ad, lap, C, cen[l][sc], n[0], n[1], n[2], n[3]);
     }
   };
@@ -772,13 +785,13 @@ __device__ __forceinline__ void marchk_impl(
 }
 
 template <typename T, int BC, int K, int DEPTH, int SW = WAVE - 2 * K, bool LW = false,
-          bool MODES = false>
+          bool MODES = false, Mask MASK = FIVE>
 __device__ __forceinline__ void marchk(
     const T* __restrict__ iCr, const T* __restrict__ iNb, const T* __restrict__ ipd,
     const T* __restrict__ ipl, T* __restrict__ oCr, T* __restrict__ oNb, T* __restrict__ opd,
     T* __restrict__ opl, int Nx, int Ny, int pitch, int strip, int chunk, int rows,
     const StepParams& P, LdsPtr lw = nullptr) {
-  marchk_impl<T, BC, K, DEPTH, SW, LW, MODES>(iCr, iNb, ipd, ipl, oCr, oNb, opd, opl, Nx, Ny, pitch,
+  marchk_impl<T, BC, K, DEPTH, SW, LW, MODES, MASK>(iCr, iNb, ipd, ipl, oCr, oNb, opd, opl, Nx, Ny, pitch,
                                        strip, chunk, rows, P, lw);
 }
 

@@ -14,7 +14,7 @@
 
 namespace pf {
 
-template <typename T, int BC, bool NINE, bool NUC, int DEPTH>
+template <typename T, int BC, Mask MASK, bool NUC, int DEPTH>
 __global__ __launch_bounds__(WAVE * WPB) void step_kernel(
     const T* __restrict__ iCr, const T* __restrict__ iNb, const T* __restrict__ ipd,
     const T* __restrict__ ipl, T* __restrict__ oCr, T* __restrict__ oNb, T* __restrict__ opd,
@@ -25,7 +25,7 @@ __global__ __launch_bounds__(WAVE * WPB) void step_kernel(
   const int b = (remap ? xcd_remap(blockIdx.x, nblocks) : (int)blockIdx.x) * WPB +
                 __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));  // wave-uniform
   if (b >= nwaves) return;  // whole wave exits; no barriers in this kernel
-  march<T, BC, NINE, NUC, DEPTH>(iCr, iNb, ipd, ipl, oCr, oNb, opd, opl, Nx, Ny, pitch,
+  march<T, BC, MASK, NUC, DEPTH>(iCr, iNb, ipd, ipl, oCr, oNb, opd, opl, Nx, Ny, pitch,
                                  b % strips, b / strips, rows, P, N, S);
 }
 
@@ -39,7 +39,7 @@ int default_rows(int nx, int ny) {
   return rows;
 }
 
-template <typename T, int BC, bool NINE, bool NUC, int DEPTH>
+template <typename T, int BC, Mask MASK, bool NUC, int DEPTH>
 static hipError_t launch_step_t(int nx, int ny, const StepParams& P, const T* iCr, const T* iNb,
                                 const T* ipd, const T* ipl, T* oCr, T* oNb, T* opd, T* opl,
                                 const NucParams& N, const Scratch& S, const TileConfig& tc,
@@ -49,7 +49,7 @@ static hipError_t launch_step_t(int nx, int ny, const StepParams& P, const T* iC
   const int strips = (Nx + STRIP - 1) / STRIP;
   const int chunks = (Ny + rows - 1) / rows;
   const int blocks = (strips * chunks + WPB - 1) / WPB;
-  hipLaunchKernelGGL((step_kernel<T, BC, NINE, NUC, DEPTH>), dim3(blocks), dim3(WAVE * WPB),
+  hipLaunchKernelGGL((step_kernel<T, BC, MASK, NUC, DEPTH>), dim3(blocks), dim3(WAVE * WPB),
                      0, st, iCr, iNb, ipd, ipl, oCr, oNb, opd, opl, Nx, Ny, nx, strips, chunks,
                      rows, tc.remap, P, N, S);
   return hipGetLastError();
@@ -63,12 +63,12 @@ static hipError_t launch_plain(int nx, int ny, const StepParams& P, const T* iCr
                                const NucParams& N, const Scratch& S, const TileConfig& tc,
                                hipStream_t st) {
   if (tc.depth == 2)
-    return launch_step_t<T, BC, false, false, 2>(nx, ny, P, iCr, iNb, ipd, ipl, oCr, oNb, opd,
+    return launch_step_t<T, BC, FIVE, false, 2>(nx, ny, P, iCr, iNb, ipd, ipl, oCr, oNb, opd,
                                                  opl, N, S, tc, st);
   if (tc.depth == 6)
-    return launch_step_t<T, BC, false, false, 6>(nx, ny, P, iCr, iNb, ipd, ipl, oCr, oNb, opd,
+    return launch_step_t<T, BC, FIVE, false, 6>(nx, ny, P, iCr, iNb, ipd, ipl, oCr, oNb, opd,
                                                  opl, N, S, tc, st);
-  return launch_step_t<T, BC, false, false, 3>(nx, ny, P, iCr, iNb, ipd, ipl, oCr, oNb, opd, opl,
+  return launch_step_t<T, BC, FIVE, false, 3>(nx, ny, P, iCr, iNb, ipd, ipl, oCr, oNb, opd, opl,
                                                N, S, tc, st);
 }
 
@@ -77,33 +77,34 @@ hipError_t launch_step(int nx, int ny, int bc, const StepParams& P, const T* iCr
                        const T* ipd, const T* ipl, T* oCr, T* oNb, T* opd, T* opl,
                        const NucParams* nuc, const Scratch& S, const TileConfig& tc,
                        hipStream_t st) {
-  const bool nine = !folded_five_point(P.m);  // the general nine-term Laplacian
   NucParams N{};
   if (nuc) N = *nuc;
-#define PF_LAUNCH(BCV, NI, NU)                                                                  \
-  return launch_step_t<T, BCV, NI, NU, 3>(nx, ny, P, iCr, iNb, ipd, ipl, oCr, oNb, opd, opl, N, \
-                                          S, tc, st)
+#define PF_LAUNCH(BCV, MASK)                                                                    \
+  do {                                                                                          \
+    if (nuc)                                                                                    \
+      return launch_step_t<T, BCV, MASK, true, 3>(nx, ny, P, iCr, iNb, ipd, ipl, oCr, oNb, opd, \
+                                                  opl, N, S, tc, st);                           \
+    if (MASK != FIVE)                                                                           \
+      return launch_step_t<T, BCV, MASK, false, 3>(nx, ny, P, iCr, iNb, ipd, ipl, oCr, oNb,     \
+                                                   opd, opl, N, S, tc, st);                     \
+    return launch_plain<T, BCV>(nx, ny, P, iCr, iNb, ipd, ipl, oCr, oNb, opd, opl, N, S, tc,    \
+                                st);                                                            \
+  } while (0)
+  const bool five = folded_five_point(P.m), nine = symmetric_nine_point(P.m);
   if (bc == 0) {
-    if (nine) {
-      if (nuc) PF_LAUNCH(0, true, true);
-      PF_LAUNCH(0, true, false);
-    }
-    if (nuc) PF_LAUNCH(0, false, true);
-    return launch_plain<T, 0>(nx, ny, P, iCr, iNb, ipd, ipl, oCr, oNb, opd, opl, N, S, tc, st);
-  } else {
-    if (nine) {
-      if (nuc) PF_LAUNCH(1, true, true);
-      PF_LAUNCH(1, true, false);
-    }
-    if (nuc) PF_LAUNCH(1, false, true);
-    return launch_plain<T, 1>(nx, ny, P, iCr, iNb, ipd, ipl, oCr, oNb, opd, opl, N, S, tc, st);
+    if (five) PF_LAUNCH(0, FIVE);
+    if (nine) PF_LAUNCH(0, NINE);
+    PF_LAUNCH(0, ANY);
   }
+  if (five) PF_LAUNCH(1, FIVE);
+  if (nine) PF_LAUNCH(1, NINE);
+  PF_LAUNCH(1, ANY);
 #undef PF_LAUNCH
 }
 
 // ---- K steps per launch (marchk, K = 2, 3 or 4) ----
 
-template <typename T, int BC, int K, int DEPTH, bool MODES>
+template <typename T, int BC, int K, int DEPTH, bool MODES, Mask MASK = FIVE>
 __global__ __launch_bounds__(WAVE * WPB) void stepk_kernel(
     const T* __restrict__ iCr, const T* __restrict__ iNb, const T* __restrict__ ipd,
     const T* __restrict__ ipl, T* __restrict__ oCr, T* __restrict__ oNb, T* __restrict__ opd,
@@ -114,8 +115,8 @@ __global__ __launch_bounds__(WAVE * WPB) void stepk_kernel(
   const int b = (remap ? xcd_remap(blockIdx.x, nblocks) : (int)blockIdx.x) * WPB +
                 __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));  // wave-uniform
   if (b >= nwaves) return;
-  marchk<T, BC, K, DEPTH, WAVE - 2 * K, false, MODES>(iCr, iNb, ipd, ipl, oCr, oNb, opd, opl, Nx,
-                                                      Ny, pitch, b % strips, b / strips, rows, P);
+  marchk<T, BC, K, DEPTH, WAVE - 2 * K, false, MODES, MASK>(
+      iCr, iNb, ipd, ipl, oCr, oNb, opd, opl, Nx, Ny, pitch, b % strips, b / strips, rows, P);
 }
 
 // Four steps: the rows behind of the four levels' windows live in LDS (8 KiB
@@ -125,7 +126,7 @@ __global__ __launch_bounds__(WAVE * WPB) void stepk_kernel(
 // on a domain full of particles (380 us before the sums of update_cell were
 // nested and its constant addends kept in vector registers), 75% of it VALU
 // issue.
-template <typename T, int BC, int DEPTH, bool MODES>
+template <typename T, int BC, int DEPTH, bool MODES, Mask MASK = FIVE>
 __global__ __launch_bounds__(WAVE * WPB) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void step4_kernel(const T* __restrict__ iCr, const T* __restrict__ iNb,
                   const T* __restrict__ ipd, const T* __restrict__ ipl, T* __restrict__ oCr,
@@ -139,9 +140,9 @@ void step4_kernel(const T* __restrict__ iCr, const T* __restrict__ iNb,
   const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));  // wave-uniform
   const int b = (remap ? xcd_remap(blockIdx.x, nblocks) : (int)blockIdx.x) * WPB + w;
   if (b >= nwaves) return;
-  marchk<T, BC, K, DEPTH, WAVE - 2 * K, true, MODES>(iCr, iNb, ipd, ipl, oCr, oNb, opd, opl, Nx,
-                                                     Ny, pitch, b % strips, b / strips, rows, P,
-                                                     (LdsPtr)win_lds + w * PER_WAVE);
+  marchk<T, BC, K, DEPTH, WAVE - 2 * K, true, MODES, MASK>(
+      iCr, iNb, ipd, ipl, oCr, oNb, opd, opl, Nx, Ny, pitch, b % strips, b / strips, rows, P,
+      (LdsPtr)win_lds + w * PER_WAVE);
 }
 
 // Chunk height of the four-step kernel from a model of its launch on
@@ -212,6 +213,15 @@ static hipError_t launch_stepk_t(int nx, int ny, const StepParams& P, const T* i
 #define PF_LAUNCH_MARCH(KERNEL)                                                                 \
   hipLaunchKernelGGL(KERNEL, dim3(blocks), dim3(WAVE * WPB), 0, st, iCr, iNb, ipd, ipl, oCr,    \
                      oNb, opd, opl, Nx, Ny, nx, strips, chunks, rows, remap, P)
+  if constexpr (K != 3) {
+    if (!folded_five_point(P.m)) {
+      if constexpr (K == 4)
+        PF_LAUNCH_MARCH((step4_kernel<T, BC, 3, false, NINE>));
+      else
+        PF_LAUNCH_MARCH((stepk_kernel<T, BC, K, 3, false, NINE>));
+      return hipGetLastError();
+    }
+  }
   if constexpr (K == 4) {
     if (rows >= MODE_ROWS)
       PF_LAUNCH_MARCH((step4_kernel<T, BC, 4, true>));

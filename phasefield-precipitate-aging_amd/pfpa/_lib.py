@@ -68,6 +68,10 @@ PROTOTYPES = {
     "pf_step3_f32": (_i, [_vp, _i, _i, _i, ctypes.POINTER(PfParams)] + [_vp] * 8 + [_vp]),
     "pf_step4_f64": (_i, [_vp, _i, _i, _i, ctypes.POINTER(PfParams)] + [_vp] * 8 + [_vp]),
     "pf_step4_f32": (_i, [_vp, _i, _i, _i, ctypes.POINTER(PfParams)] + [_vp] * 8 + [_vp]),
+    "pf_advance_f64": (_i, [_vp, _i, _i, _i, ctypes.POINTER(PfParams), ctypes.POINTER(_vp),
+                            ctypes.POINTER(_vp), ctypes.c_uint64, _i, ctypes.POINTER(_i), _vp]),
+    "pf_advance_f32": (_i, [_vp, _i, _i, _i, ctypes.POINTER(PfParams), ctypes.POINTER(_vp),
+                            ctypes.POINTER(_vp), ctypes.c_uint64, _i, ctypes.POINTER(_i), _vp]),
     "pf_ctx_set_tile2": (_i, [_vp, _i, _i]),
     "pf_default_rows2": (_i, [_i, _i, _i]),
     "pf_ctx_set_tile3": (_i, [_vp, _i, _i]),

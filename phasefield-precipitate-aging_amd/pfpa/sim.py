@@ -1,6 +1,6 @@
-"""Native stepping loop over the C-ABI.  Steps run up to four per launch
-(the temporally blocked kernels) wherever no step of the group is a
-nucleation step; nucleation steps, the ones the reference's schedule selects
+"""Native stepping loop over the C-ABI.  The steps between two nucleation
+steps are one call (pf_advance_*), which runs up to four per launch (the
+temporally blocked kernels); nucleation steps, the ones the reference's schedule selects
 (kernel_time % nuc_interval == 0, src/main.cpp:307-316), run one per launch
 with the nucleation pass fused."""
 import ctypes
@@ -154,7 +154,12 @@ class Simulation:
         self._stepk = {2: lib().pf_step2_f64 if f64 else lib().pf_step2_f32,
                        3: lib().pf_step3_f64 if f64 else lib().pf_step3_f32,
                        4: lib().pf_step4_f64 if f64 else lib().pf_step4_f32}
+        self._advance = lib().pf_advance_f64 if f64 else lib().pf_advance_f32
         self.steps_per_launch = default_steps_per_launch(setup, dtype, steps_per_launch)
+        # other masks have no pf_step2..4_* entry points, but symmetric
+        # nine-point ones run four steps per launch all the same (pf_advance_*)
+        self._group_other_masks = (steps_per_launch is None and
+                                   not M.symmetric_five_point(setup.mask))
         self._summ = lib().pf_summarize_f64 if dtype == torch.float64 else lib().pf_summarize_f32
 
     def set_tile(self, rows, remap=1, depth=0):
@@ -226,29 +231,32 @@ class Simulation:
 
     def step(self, n=1):
         st = ctypes.c_void_p(self.stream.cuda_stream)
-        plan = iter_launches(self.steps_done, n, self.steps_per_launch,
-                             self.nuc_every if self.nucleation else 0)
-        for k, nucleate in plan:
+        end = self.steps_done + n
+        while self.steps_done < end:
             a, b = self.a, self.b
             t = self.steps_done
-            if k > 1:
-                check(self._stepk[k](self.ctx, self.nx, self.ny, self.s.bc, ctypes.byref(self.P),
-                                     _ptr(a[0]), _ptr(a[1]), _ptr(a[2]), _ptr(a[3]),
-                                     _ptr(b[0]), _ptr(b[1]), _ptr(b[2]), _ptr(b[3]), st),
-                      "pf_step%d" % k)
-                done = k
-            else:
-                nuc = None
-                if nucleate:
-                    self.N.call = t // self.nuc_every
-                    nuc = ctypes.byref(self.N)
+            if self.nucleation and t % self.nuc_every == 0:
+                self.N.call = t // self.nuc_every
                 check(self._step(self.ctx, self.nx, self.ny, self.s.bc, ctypes.byref(self.P),
                                  _ptr(a[0]), _ptr(a[1]), _ptr(a[2]), _ptr(a[3]),
-                                 _ptr(b[0]), _ptr(b[1]), _ptr(b[2]), _ptr(b[3]), nuc, st),
-                      "pf_step")
-                done = 1
-            self.a, self.b = self.b, self.a
-            self.steps_done += done
+                                 _ptr(b[0]), _ptr(b[1]), _ptr(b[2]), _ptr(b[3]),
+                                 ctypes.byref(self.N), st), "pf_step")
+                self.a, self.b = b, a
+                self.steps_done += 1
+                continue
+            # the steps up to the next nucleation step in one native call
+            k = end - t
+            if self.nucleation:
+                k = min(k, self.nuc_every - t % self.nuc_every)
+            in_b = ctypes.c_int()
+            most = 4 if self._group_other_masks else self.steps_per_launch
+            check(self._advance(self.ctx, self.nx, self.ny, self.s.bc, ctypes.byref(self.P),
+                                (ctypes.c_void_p * 4)(*[x.data_ptr() for x in a]),
+                                (ctypes.c_void_p * 4)(*[x.data_ptr() for x in b]), k,
+                                most, ctypes.byref(in_b), st), "pf_advance")
+            if in_b.value:
+                self.a, self.b = b, a
+            self.steps_done += k
 
     def fields(self):
         """The current fields as FP64 arrays, compositions in absolute units."""
