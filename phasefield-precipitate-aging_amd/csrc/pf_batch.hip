@@ -12,11 +12,11 @@
 //
 // Per launch: step kernel (on every active job's strips, reading the job's
 // current set and writing the other: pf::marchk when the job advances two or
-// three steps this launch, pf::march for one), then the nucleation kernel
-// (jobs whose schedule is due on the last step of the launch; centre-only
-// embeds), then a one-block kernel that advances every active job's step
-// counter, retires jobs that reached their target and decides each job's next
-// advance.  A job advances k steps in a launch (k up to the batch's steps per
+// three steps this launch, pf::march for one), then, if any job of the mix has
+// nucleation, the nucleation kernel (jobs whose schedule is due on the last
+// step of the launch; centre-only embeds).  The last block to finish, of the
+// step kernel or of a nucleation kernel with work to do, advances every active job's step counter, retires jobs that
+// reached their target and decides each job's next advance.  A job advances k steps in a launch (k up to the batch's steps per
 // launch) when k steps remain and no nucleation step falls before the last of
 // them.
 // A job's arithmetic and tiling depend only on the job, so its result is the
@@ -60,12 +60,75 @@ struct BatchHeader {
   // launches), one 128-byte line each: on one shared line the eight XCDs'
   // atomics contend and the FP64 batch ran 1.4% slower
   unsigned int next_task[8][32];
+  // blocks of a kernel that have finished: by blockIdx % 8 ([x][0], a line
+  // each), then of these eight groups
+  unsigned int blocks_done[8][32];
+  unsigned int groups_done;
+  int nuc_now;  // the nucleation kernel of this launch has work
 };
 
 // the last step of this launch is one of the job's nucleation steps
 __host__ __device__ __forceinline__ bool nuc_due(const BatchJob& J) {
   return J.active && !J.held && J.nuc_every > 0 &&
          (J.step + (uint64_t)J.adv - 1) % (uint64_t)J.nuc_every == 0;
+}
+
+// the job's advance in the next launch (a multi-step launch never has a
+// nucleation step before its last step)
+__host__ __device__ __forceinline__ int next_adv(const BatchJob& J) {
+  int k = 1;
+  while (k < J.max_adv && J.step + k + 1 <= J.target &&
+         !(J.nuc_every > 0 && (J.step + k - 1) % (uint64_t)J.nuc_every == 0))
+    k++;
+  return k;
+}
+
+// Whether the calling block is the kernel's last to get here (the grid is a
+// multiple of 8 blocks).  The count needs no fence (one by each block writes
+// back its XCD's L2: 30 us per launch): a block has used every job entry and
+// task claim it read when it counts itself, the entries are written by no one
+// before, and the next launch sees what the last block writes.  Eight counters
+// first: a thousand atomics on one took 14 us.
+__device__ __forceinline__ bool last_block(BatchHeader* hdr) {
+  __shared__ int last;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    last = 0;
+    unsigned int* group = &hdr->blocks_done[blockIdx.x & 7][0];
+    if (atomicAdd(group, 1u) == (gridDim.x >> 3) - 1) {
+      *group = 0u;
+      if (atomicAdd(&hdr->groups_done, 1u) == 7u) {
+        hdr->groups_done = 0u;
+        last = 1;
+      }
+    }
+  }
+  __syncthreads();
+  return last != 0;
+}
+
+// By one block, when all others are done with the jobs: advance every active
+// job by this launch's steps, flip its buffer parity, retire it at its target,
+// decide its next advance, and record whether any job is due at the next
+// launch.  (As a kernel of one block after the others this cost 4.5 us and a
+// gap per launch beside 50-90 us of steps.)
+__device__ __forceinline__ void advance_jobs(BatchJob* jobs, BatchHeader* hdr) {
+  int due = 0;
+  for (int j = threadIdx.x; j < hdr->njobs; j += blockDim.x) {
+    BatchJob& J = jobs[j];
+    if (J.active && !J.held) {
+      J.step += J.adv;
+      J.parity ^= 1;
+      if (J.step >= J.target) J.active = 0;
+      J.adv = next_adv(J);
+      due |= nuc_due(J) ? 1 : 0;
+    }
+  }
+  due = __syncthreads_or(due);
+  if (threadIdx.x == 0) {
+    hdr->any_due = due;
+    hdr->nuc_now = 0;
+  }
 }
 
 constexpr int BATCH_RB = 16;  // reduction blocks per job
@@ -89,12 +152,14 @@ __device__ __forceinline__ void xcd_range(int total, int& first, int& last, int&
 // claims its next task from the XCD's counter (one atomic, by lane 0), so
 // waves that draw short tasks take more of them.  The claim for the next
 // task is issued before the current task runs and read after it; waves with
-// no first task exit without touching the counter.
+// no first task leave the counter alone.  `table` is `jobs`, for the last
+// block to write.
 template <typename T, int DEPTH>
 __global__ __launch_bounds__(WAVE * WPB) void batch_step_kernel(const BatchJob* __restrict__ jobs,
                                                                 const int* __restrict__ wave_job,
                                                                 BatchHeader* __restrict__ hdr,
-                                                                T* __restrict__ pool) {
+                                                                T* __restrict__ pool,
+                                                                BatchJob* table) {
   int first, last, nwaves, w;
   xcd_range(hdr->total_waves, first, last, nwaves, w);
   unsigned int* ctr = &hdr->next_task[blockIdx.x & 7][0];
@@ -137,21 +202,17 @@ __global__ __launch_bounds__(WAVE * WPB) void batch_step_kernel(const BatchJob* 
 #undef PF_BATCH_MARCH
     w = first + nwaves + (int)__builtin_amdgcn_readfirstlane(next);
   }
+  if (!last_block(hdr)) return;
+  if (threadIdx.x < 8) hdr->next_task[threadIdx.x][0] = 0u;  // the next step launch claims from 0
+  if (hdr->any_due) {  // the nucleation kernel comes first
+    if (threadIdx.x == 0) hdr->nuc_now = 1;
+  } else {
+    advance_jobs(table, hdr);
+  }
 }
 
 // Nucleation on the new fields of the jobs whose schedule is due on the last
-// step of this launch (src/main.cpp:307-316 schedule, centre-only embeds);
-// then batch_advance_kernel advances the step counters and picks each job's
-// next advance (a multi-step launch never has a nucleation step before its
-// last step).
-__host__ __device__ __forceinline__ int next_adv(const BatchJob& J) {
-  int k = 1;
-  while (k < J.max_adv && J.step + k + 1 <= J.target &&
-         !(J.nuc_every > 0 && (J.step + k - 1) % (uint64_t)J.nuc_every == 0))
-    k++;
-  return k;
-}
-
+// step of this launch (src/main.cpp:307-316 schedule, centre-only embeds).
 template <typename T>
 __global__ __launch_bounds__(WAVE * WPB) void batch_nuc_kernel(
     BatchJob* __restrict__ jobs, const int* __restrict__ wave_job, BatchHeader* __restrict__ hdr,
@@ -160,8 +221,8 @@ __global__ __launch_bounds__(WAVE * WPB) void batch_nuc_kernel(
   xcd_range(hdr->total_waves, first, last, stride, w);
   const int lane = threadIdx.x & (WAVE - 1);
   // launches without a due job (all but one in nuc_every / steps per launch)
-  // skip the scan of the wave table
-  if (!hdr->any_due) return;
+  // end here
+  if (!hdr->nuc_now) return;
   for (; w < last; w += stride) {
     const int j = __builtin_amdgcn_readfirstlane(wave_job[w]);
     const BatchJob& J = jobs[j];
@@ -199,28 +260,7 @@ __global__ __launch_bounds__(WAVE * WPB) void batch_nuc_kernel(
       }
     }
   }
-}
-
-// One block after the nucleation kernel (stream order): advance every active
-// job by this launch's steps, flip its buffer parity, retire it at its target,
-// decide its next advance, and record whether any job is due at the next
-// launch.
-__global__ __launch_bounds__(256) void batch_advance_kernel(BatchJob* __restrict__ jobs,
-                                                            BatchHeader* __restrict__ hdr) {
-  int due = 0;
-  for (int j = threadIdx.x; j < hdr->njobs; j += blockDim.x) {
-    BatchJob& J = jobs[j];
-    if (J.active && !J.held) {
-      J.step += J.adv;
-      J.parity ^= 1;
-      if (J.step >= J.target) J.active = 0;
-      J.adv = next_adv(J);
-      due |= nuc_due(J) ? 1 : 0;
-    }
-  }
-  due = __syncthreads_or(due);
-  if (threadIdx.x == 0) hdr->any_due = due;
-  if (threadIdx.x < 8) hdr->next_task[threadIdx.x][0] = 0u;  // the next step launch claims from 0
+  if (last_block(hdr)) advance_jobs(jobs, hdr);
 }
 
 // per-job deterministic compensated sums: block (j, r) reduces rows
@@ -318,6 +358,8 @@ struct pf_batch {
   // graph
   hipGraphExec_t graph = nullptr;
   int graph_steps = 0, graph_depth = 0;
+  bool graph_nuc = false;
+  bool nuc = false;  // some job of the committed mix has nucleation
 };
 
 namespace {
@@ -396,23 +438,21 @@ hipError_t launch_batch_step(pf_batch* b, hipStream_t st) {
   switch (b->depth) {
     case 2:
       hipLaunchKernelGGL((pf::batch_step_kernel<T, 2>), grid, block, 0, st, b->d_jobs,
-                         b->d_wave_job, b->d_hdr, pool);
+                         b->d_wave_job, b->d_hdr, pool, b->d_jobs);
       break;
     case 6:
       hipLaunchKernelGGL((pf::batch_step_kernel<T, 6>), grid, block, 0, st, b->d_jobs,
-                         b->d_wave_job, b->d_hdr, pool);
+                         b->d_wave_job, b->d_hdr, pool, b->d_jobs);
       break;
     default:
       hipLaunchKernelGGL((pf::batch_step_kernel<T, 3>), grid, block, 0, st, b->d_jobs,
-                         b->d_wave_job, b->d_hdr, pool);
+                         b->d_wave_job, b->d_hdr, pool, b->d_jobs);
   }
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(pf::batch_nuc_kernel<T>, grid, block, 0, st, b->d_jobs, b->d_wave_job,
-                     b->d_hdr, pool);
-  e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(pf::batch_advance_kernel, dim3(1), dim3(256), 0, st, b->d_jobs, b->d_hdr);
+  if (e != hipSuccess || !b->nuc) return e;
+  // a quarter of the blocks: nearly every launch only looks at one flag
+  hipLaunchKernelGGL(pf::batch_nuc_kernel<T>, dim3(b->grid_blocks / 32 * 8), block, 0, st,
+                     b->d_jobs, b->d_wave_job, b->d_hdr, pool);
   return hipGetLastError();
 }
 
@@ -662,9 +702,16 @@ int pf_batch_commit(pf_batch* b) {
   h.njobs = (int)b->jobs.size();
   for (int x = 0; x < 8; x++) h.next_task[x][0] = 0u;
   h.pad = 0u;
+  for (int x = 0; x < 8; x++) h.blocks_done[x][0] = 0u;
+  h.groups_done = 0u;
+  h.nuc_now = 0;
   h.any_due = 0;
+  b->nuc = false;
   for (size_t j = 0; j < b->jobs.size(); j++)
-    if (b->slot_live[j] && pf::nuc_due(b->jobs[j])) h.any_due = 1;
+    if (b->slot_live[j]) {
+      if (pf::nuc_due(b->jobs[j])) h.any_due = 1;
+      if (b->jobs[j].active && !b->jobs[j].held && b->jobs[j].nuc_every > 0) b->nuc = true;
+    }
   if ((e = hipMemcpy(b->d_hdr, &h, sizeof(h), hipMemcpyHostToDevice)) != hipSuccess)
     return bhip(e, "upload header");
   for (size_t j = 0; j < b->jobs.size(); j++) b->slot_on_device[j] = b->slot_live[j];
@@ -679,7 +726,8 @@ int pf_batch_run(pf_batch* b, int launches, int per_graph) {
   hipError_t e;
   int done = 0;
   if (per_graph > 1) {
-    if (!b->graph || b->graph_steps != per_graph || b->graph_depth != b->depth) {
+    if (!b->graph || b->graph_steps != per_graph || b->graph_depth != b->depth ||
+        b->graph_nuc != b->nuc) {
       if (b->graph) {
         (void)hipGraphExecDestroy(b->graph);
         b->graph = nullptr;
@@ -697,6 +745,7 @@ int pf_batch_run(pf_batch* b, int launches, int per_graph) {
       if (e != hipSuccess) return bhip(e, "instantiate graph");
       b->graph_steps = per_graph;
       b->graph_depth = b->depth;
+      b->graph_nuc = b->nuc;
     }
     for (; done + per_graph <= launches; done += per_graph)
       if ((e = hipGraphLaunch(b->graph, b->stream)) != hipSuccess) return bhip(e, "graph launch");
