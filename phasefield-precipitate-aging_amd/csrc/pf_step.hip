@@ -145,6 +145,76 @@ void step4_kernel(const T* __restrict__ iCr, const T* __restrict__ iNb,
       (LdsPtr)win_lds + w * PER_WAVE);
 }
 
+// Four steps on a small grid.  A march takes some ten iterations of four
+// dependent levels however short its chunks are, and a small grid has too few
+// waves to hide them: 7 us of latency.  Here a block takes a tile of TX x TY
+// output cells with a halo of four, one cell per thread, and all threads go
+// through the four levels together, exchanging a level's values through LDS
+// (two buffers, so one barrier per level).  The cells of the halo are computed
+// by every block that needs them, (TX + 8)(TY + 8) / (TX TY) times the work,
+// which is why larger grids march.
+template <typename T, int BC, int TX, int TY>
+__global__ __launch_bounds__((TX + 8) * (TY + 8)) void tile4_kernel(
+    const T* __restrict__ iCr, const T* __restrict__ iNb, const T* __restrict__ ipd,
+    const T* __restrict__ ipl, T* __restrict__ oCr, T* __restrict__ oNb, T* __restrict__ opd,
+    T* __restrict__ opl, int Nx, int Ny, int pitch, int tiles_x, StepParams P) {
+  constexpr int K = 4, W = TX + 2 * K, H = TY + 2 * K, CELLS = W * H;
+  __shared__ double buf[2][4][CELLS];
+  const int b = xcd_remap(blockIdx.x, gridDim.x);
+  const int tid = threadIdx.x;
+  const int tx = tid % W, ty = tid / W;
+  const int gx = (b % tiles_x) * TX + tx - K, gy = (b / tiles_x) * TY + ty - K;
+  Raw<T> r;
+  load_row(r, iCr, iNb, ipd, ipl, (size_t)(1 + bc_map<BC>(gy, Ny)) * pitch * sizeof(T),
+           (uint32_t)(1 + bc_map<BC>(gx, Nx)) * (uint32_t)sizeof(T));
+  // neighbours; on the tile's rim, whose values no output needs, the cell itself
+  const int w = tx > 0 ? tid - 1 : tid, e = tx < W - 1 ? tid + 1 : tid;
+  const int s = ty > 0 ? tid - W : tid, n = ty < H - 1 ? tid + W : tid;
+  const Addends ad = addends(P);
+  Point v;
+  Centre c;
+  derive<T>(ad, r, v, c);
+#pragma unroll
+  for (int l = 0; l < K; l++) {
+    double(*f)[CELLS] = buf[l & 1];
+    f[0][tid] = v.pd;
+    f[1][tid] = v.pl;
+    f[2][tid] = v.mu0;
+    f[3][tid] = v.mu1;
+    __syncthreads();
+    const double own[4] = {v.pd, v.pl, v.mu0, v.mu1};
+    double lap[4], o[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) lap[q] = five_point(P.m, f[q][s], f[q][w], own[q], f[q][e], f[q][n]);
+    update_cell(P, ad, lap, v, c, o[0], o[1], o[2], o[3]);
+    if (l < K - 1) {
+      derive<T>(ad, Raw<T>{(T)o[0], (T)o[1], (T)o[2], (T)o[3]}, v, c);
+    } else if (tx >= K && tx < K + TX && ty >= K && ty < K + TY && gx < Nx && gy < Ny) {
+      store4(oCr, oNb, opd, opl, (size_t)(1 + gy) * pitch + 1 + gx, o[0], o[1], o[2], o[3]);
+      store_ghost_images<T, BC>(oCr, oNb, opd, opl, gx, gy, Nx, Ny, pitch, o[0], o[1], o[2],
+                                o[3]);
+    }
+  }
+}
+
+// Side of the tiles of a small grid, 0 where it marches.  A tile of 8, 12 or 16
+// is 4, 7 or 9 waves; with one tile per CU (256) the smallest that covers the
+// grid is the fastest, then two of 12 per CU, then two of 16.  us per launch
+// (FP64, back to back), march / tiles of 8 / 12 / 16: 128^2 7.6 / 4.3 / 4.9 /
+// 5.5, 192^2 7.7 / 5.6 / 4.9 / 5.6, 256^2 8.8 / 6.5 / 6.2 / 5.7, 131 x 515
+// 8.8 / 7.0 / 6.2 / 7.3, 340^2 10.1 / 9.3 / 9.1 / 7.5, 384^2 10.2 / 10.4 / 9.4
+// / 10.1, 512^2 (14 / - / - / 14.3) and up the march.
+static int tile_side(int Nx, int Ny) {
+  auto tiles = [&](int side) {
+    return (long)((Nx + side - 1) / side) * ((Ny + side - 1) / side);
+  };
+  for (int side : {8, 12, 16})
+    if (tiles(side) <= 256) return side;
+  for (int side : {12, 16})
+    if (tiles(side) <= 512) return side;
+  return 0;
+}
+
 // Chunk height of the four-step kernel from a model of its launch on
 // MI355X: 256 CUs x 4 SIMDs hold 2048 waves at two waves per SIMD.  A wave's
 // time is proportional to its rows plus the 3 rows (K - 1) its levels
@@ -223,6 +293,22 @@ static hipError_t launch_stepk_t(int nx, int ny, const StepParams& P, const T* i
     }
   }
   if constexpr (K == 4) {
+    const int tile = rows_cfg == 0 ? tile_side(Nx, Ny) : 0;
+    if (tile) {
+      const int tiles_x = (Nx + tile - 1) / tile, tiles = tiles_x * ((Ny + tile - 1) / tile);
+      const dim3 threads((tile + 8) * (tile + 8));
+#define PF_LAUNCH_TILE(S)                                                                       \
+  hipLaunchKernelGGL((tile4_kernel<T, BC, S, S>), dim3(tiles), threads, 0, st, iCr, iNb, ipd,   \
+                     ipl, oCr, oNb, opd, opl, Nx, Ny, nx, tiles_x, P)
+      if (tile == 8)
+        PF_LAUNCH_TILE(8);
+      else if (tile == 12)
+        PF_LAUNCH_TILE(12);
+      else
+        PF_LAUNCH_TILE(16);
+#undef PF_LAUNCH_TILE
+      return hipGetLastError();
+    }
     if (rows >= MODE_ROWS)
       PF_LAUNCH_MARCH((step4_kernel<T, BC, 4, true>));
     else
