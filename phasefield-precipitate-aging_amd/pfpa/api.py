@@ -86,7 +86,8 @@ class CudaData:
         self.nuc_calls = 0
         self.pending = []
         self.group = 4        # steps per launch of grouped device_evolution calls
-        self.queued = 0       # steps recorded and not yet run (0..2)
+        self.queued = 0       # steps recorded and not yet run (0..7)
+        self.queued_mask = b""  # the mask (bytes) the first of them was recorded with
         self.first = None     # (old, new, alpha, dt, nx, ny) of the first of them
 
 
@@ -219,11 +220,19 @@ def device_laplacian_boundaries(dev, nx, ny, nm, bx, by):
     _record(dev, "laplacian_boundaries")
 
 
-_FIELDS = ("conc_Cr", "conc_Nb", "phi_del", "phi_lav")
+def _old_fields(dev):
+    return dev.conc_Cr_old, dev.conc_Nb_old, dev.phi_del_old, dev.phi_lav_old
 
 
-def _fields(dev, which):
-    return tuple(getattr(dev, f + which) for f in _FIELDS)
+def _new_fields(dev):
+    return dev.conc_Cr_new, dev.conc_Nb_new, dev.phi_del_new, dev.phi_lav_new
+
+
+def _same_arrays(a, b):
+    for x, y in zip(a, b):
+        if x is not y and x.data_ptr() != y.data_ptr():
+            return False
+    return True
 
 
 def _launch(dev, fn, nx, ny, alpha, dt, old, new, *extra):
@@ -282,8 +291,12 @@ def device_evolution(dev, nx, ny, nm, bx, by, alpha, dt):
     """src/discretization.cu:982-1020: one fused step *_old -> *_new, grouped
     with the calls around it (see the module docstring)."""
     dev.pending.clear()
-    old, new = _fields(dev, "_old"), _fields(dev, "_new")
-    five_point = M.symmetric_five_point(dev.params.mask)
+    old, new = _old_fields(dev), _new_fields(dev)
+    # the first step of a group looks at the mask, the others at whether it is
+    # still that one: a driver's loop over a small grid is bound by this function
+    mask = bytes(dev.params.mask)
+    five_point = (mask == dev.queued_mask if dev.queued else False) or \
+        M.symmetric_five_point(dev.params.mask)
     if dev.group == 1 or not five_point or nx < 5 or ny < 5:
         device_flush(dev)
         _launch(dev, lib().pf_step_f64, nx, ny, alpha, dt, old, new, None)
@@ -291,12 +304,12 @@ def device_evolution(dev, nx, ny, nm, bx, by, alpha, dt):
     if dev.queued:
         f_old, f_new, f_alpha, f_dt, f_nx, f_ny = dev.first
         want_old, want_new = (f_new, f_old) if dev.queued % 2 else (f_old, f_new)
-        same = (lambda a, b: all(x.data_ptr() == y.data_ptr() for x, y in zip(a, b)))
-        if not (same(old, want_old) and same(new, want_new) and (alpha, dt, nx, ny) ==
-                (f_alpha, f_dt, f_nx, f_ny)):
+        if not (_same_arrays(old, want_old) and _same_arrays(new, want_new) and
+                (alpha, dt, nx, ny) == (f_alpha, f_dt, f_nx, f_ny)):
             device_flush(dev)
     if not dev.queued:
         dev.first = (old, new, alpha, dt, nx, ny)
+        dev.queued_mask = mask
     dev.queued += 1
     if dev.queued == group_size(dev.group, nx, ny):
         device_flush(dev)
