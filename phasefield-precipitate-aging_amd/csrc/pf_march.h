@@ -583,6 +583,10 @@ __device__ __forceinline__ void march(
 //    potentials exchanged.
 //  - DENSE: the general case, at the cost of the test (seven operations per
 //    row of some 430).
+// With FAIR, a wave's priority falls by quarters of its chunk.  The older of
+// the two waves of a SIMD otherwise wins every issue slot, ends early and
+// leaves the other to run alone at two thirds of the pair's rate.
+//
 // Every mode gives the bits of DENSE: StepParams::matrix_ok says (from bounds
 // on the coefficients) that a step multiplies |phi| < TINY by 16 at most, that
 // compositions below X_MATRIX keep every product finite (so 0 * G is 0), and
@@ -597,7 +601,8 @@ __device__ __forceinline__ bool matrix_row(const Raw<T>& r) {
 __device__ __forceinline__ int set_bits(float v) { return __float_as_int(v); }
 __device__ __forceinline__ int set_bits(double v) { return __double2loint(v) | __double2hiint(v); }
 
-template <typename T, int BC, int K, int DEPTH, int SW, bool LW, bool MODES, Mask MASK>
+template <typename T, int BC, int K, int DEPTH, int SW, bool LW, bool MODES, Mask MASK,
+          bool FAIR>
 __device__ __forceinline__ void marchk_impl(
     const T* __restrict__ iCr, const T* __restrict__ iNb, const T* __restrict__ ipd,
     const T* __restrict__ ipl, T* __restrict__ oCr, T* __restrict__ oNb, T* __restrict__ opd,
@@ -751,6 +756,16 @@ __device__ __forceinline__ void marchk_impl(
 
   // ---- main loop: iteration t = 2K + i, output row y = y0 + i
   for (int ib = 0;; ib += UNROLL) {
+    if constexpr (FAIR) {
+      if (4 * ib < nrows)
+        __builtin_amdgcn_s_setprio(3);
+      else if (2 * ib < nrows)
+        __builtin_amdgcn_s_setprio(2);
+      else if (4 * ib < 3 * nrows)
+        __builtin_amdgcn_s_setprio(1);
+      else
+        __builtin_amdgcn_s_setprio(0);
+    }
 #pragma unroll
     for (int k = 0; k < UNROLL; k++) {
       if (ib + k >= nrows) return;
@@ -785,14 +800,14 @@ __device__ __forceinline__ void marchk_impl(
 }
 
 template <typename T, int BC, int K, int DEPTH, int SW = WAVE - 2 * K, bool LW = false,
-          bool MODES = false, Mask MASK = FIVE>
+          bool MODES = false, Mask MASK = FIVE, bool FAIR = false>
 __device__ __forceinline__ void marchk(
     const T* __restrict__ iCr, const T* __restrict__ iNb, const T* __restrict__ ipd,
     const T* __restrict__ ipl, T* __restrict__ oCr, T* __restrict__ oNb, T* __restrict__ opd,
     T* __restrict__ opl, int Nx, int Ny, int pitch, int strip, int chunk, int rows,
     const StepParams& P, LdsPtr lw = nullptr) {
-  marchk_impl<T, BC, K, DEPTH, SW, LW, MODES, MASK>(iCr, iNb, ipd, ipl, oCr, oNb, opd, opl, Nx, Ny, pitch,
-                                       strip, chunk, rows, P, lw);
+  marchk_impl<T, BC, K, DEPTH, SW, LW, MODES, MASK, FAIR>(
+      iCr, iNb, ipd, ipl, oCr, oNb, opd, opl, Nx, Ny, pitch, strip, chunk, rows, P, lw);
 }
 
 }  // namespace pf

@@ -126,7 +126,7 @@ __global__ __launch_bounds__(WAVE * WPB) void stepk_kernel(
 // on a domain full of particles (380 us before the sums of update_cell were
 // nested and its constant addends kept in vector registers), 75% of it VALU
 // issue.
-template <typename T, int BC, int DEPTH, bool MODES, Mask MASK = FIVE>
+template <typename T, int BC, int DEPTH, bool MODES, Mask MASK = FIVE, bool FAIR = false>
 __global__ __launch_bounds__(WAVE * WPB) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void step4_kernel(const T* __restrict__ iCr, const T* __restrict__ iNb,
                   const T* __restrict__ ipd, const T* __restrict__ ipl, T* __restrict__ oCr,
@@ -140,7 +140,7 @@ void step4_kernel(const T* __restrict__ iCr, const T* __restrict__ iNb,
   const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));  // wave-uniform
   const int b = (remap ? xcd_remap(blockIdx.x, nblocks) : (int)blockIdx.x) * WPB + w;
   if (b >= nwaves) return;
-  marchk<T, BC, K, DEPTH, WAVE - 2 * K, true, MODES, MASK>(
+  marchk<T, BC, K, DEPTH, WAVE - 2 * K, true, MODES, MASK, FAIR>(
       iCr, iNb, ipd, ipl, oCr, oNb, opd, opl, Nx, Ny, pitch, b % strips, b / strips, rows, P,
       (LdsPtr)win_lds + w * PER_WAVE);
 }
@@ -253,6 +253,18 @@ static int rows4_model(int strips, int Ny) {
 //   FP32 8192^2, 48 rows, three steps: 790 / 567, 802 / 818.
 constexpr int MODE_ROWS = 32;
 
+// Whether the four-step launch shares its SIMDs fairly (FAIR, pf_march.h): where
+// all of it is resident at once, two waves on most SIMDs, and the chunks are
+// long enough to be cut in quarters.  us per launch without / with: 1400 x 1100
+// FP32, 14 rows, 36.7 / 34.6; FP64 1021 x 1543, 15 rows, 40.0 / 39.3; 1600 x
+// 1300, 21 rows, 47.9 / 46.8; 2048 x 1536, 28 rows, 65.7 / 64.5.  With later
+// rounds the waves are staggered anyway and the rule holds the old ones back
+// (4096^2, 60 rows: 329 / 357), and on chunks of one trip it holds back the
+// prologues (700^2, 6 rows: 17.9 / 18.9).
+static bool fair_shares(long waves, int rows) {
+  return waves > 1024 && waves <= 2048 && rows >= 12;
+}
+
 int default_rows_k(int k, int nx, int ny, int storage_bytes) {
   // The intermediate levels recompute (K-1)K rows per chunk in all, so chunks
   // are longer than the one-step kernel's while the grid still fills the chip.
@@ -311,6 +323,8 @@ static hipError_t launch_stepk_t(int nx, int ny, const StepParams& P, const T* i
     }
     if (rows >= MODE_ROWS)
       PF_LAUNCH_MARCH((step4_kernel<T, BC, 4, true>));
+    else if (DEPTH == 3 && fair_shares((long)strips * chunks, rows))
+      PF_LAUNCH_MARCH((step4_kernel<T, BC, 3, false, FIVE, true>));
     else
       PF_LAUNCH_MARCH((step4_kernel<T, BC, DEPTH, false>));
   } else if constexpr (K == 3 && sizeof(T) == sizeof(float)) {

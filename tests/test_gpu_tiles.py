@@ -1,6 +1,8 @@
 """The four-step kernel's tiles on small grids (sides 8, 12 and 16, one cell
 per thread) against one-step launches: grids at the edges of a tile, of each
-tile size's range and beyond it, both boundary modes and storage types."""
+tile size's range and beyond it, where the march runs (the last two with all
+of its waves resident and sharing their SIMDs fairly), both boundary modes and
+storage types."""
 import ctypes
 
 import numpy as np
@@ -15,7 +17,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("shape", [(4, 4), (7, 5), (8, 16), (9, 17), (128, 128), (129, 128),
                                    (192, 191), (193, 192), (255, 256), (257, 256), (5, 2000),
-                                   (1999, 6), (264, 263), (362, 355), (365, 367)])
+                                   (1999, 6), (264, 263), (362, 355), (365, 367),
+                                   (1021, 1543), (1400, 1100)])
 @pytest.mark.parametrize("bc", [0, 1])
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 def test_tiles_match_one_step_launches(gpu, dtype, bc, shape):
