@@ -285,8 +285,9 @@ def plain_section(args, dtype_name="f64"):
     nuc_every = sim.nuc_every
     sim.close()
     tname = "double" if f64 else "float"
-    kname = {4: "pf::step4_kernel<%s, 1, 3>" % tname, 3: "pf::stepk_kernel<%s, 1, 3, 3>" % tname,
-             2: "pf::stepk_kernel<%s, 1, 2, 3>" % tname}
+    kname = {4: "pf::step4_kernel<%s, 1, 4, true>" % tname,
+             3: "pf::stepk_kernel<%s, 1, 3, 3, %s>" % (tname, "false" if f64 else "true"),
+             2: "pf::stepk_kernel<%s, 1, 2, 3, false>" % tname}
     valu_us = load_valu_issue(kname[K]) if N == 4096 else None
     words = {1: "one", 2: "two", 3: "three", 4: "four"}
     others = {"%s_step_kernel" % words[k]:
@@ -324,8 +325,10 @@ def plain_section(args, dtype_name="f64"):
             "kernel_us_per_step": kernK_s / K * 1e6,
             "note": "temporal blocking: one read and one write of the fields per launch "
                     "carry %d cell-updates per cell, so frac falls as K rises while the time "
-                    "per step falls; the launch is bound by FP64 arithmetic at two waves per "
-                    "SIMD (valu_issue_frac), not by HBM" % K,
+                    "per step falls; this workload holds no precipitate, so most rows need "
+                    "neither phase update nor a solve of their own and the launch is bound "
+                    "by its memory traffic (a domain full of particles: by FP64 arithmetic)"
+                    % K,
             **others,
         },
     }
