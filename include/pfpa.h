@@ -273,7 +273,10 @@ int pf_mobility_divergence_f64(int nx, int ny, double dx, double dy, const pf_mo
 int pf_default_rows(int nx, int ny);
 /* Tile of the two-step (three-, four-step) kernel: rows per chunk (0 =
  * heuristic) and prefetch depth (2, 3, 6; 0 = 3).  pf_default_rows2 (3, 4) is
- * its heuristic for storage PF_STORAGE_F64 or PF_STORAGE_F32. */
+ * its heuristic for storage PF_STORAGE_F64 or PF_STORAGE_F32.  Four steps (and
+ * FP32 three) with chunks of 32 rows and more keep a depth of their own, and so
+ * do nine-point masks; with rows = 0 four steps on a small grid run by square
+ * tiles, without chunks.  The results do not depend on any of these. */
 int pf_ctx_set_tile2(pf_ctx* ctx, int rows, int depth);
 int pf_default_rows2(int nx, int ny, int storage);
 int pf_ctx_set_tile3(pf_ctx* ctx, int rows, int depth);
@@ -331,7 +334,7 @@ int pf_batch_remove(pf_batch* batch, int job_id);
 /* Publish admissions/removals to the device tables (done by pf_batch_run too). */
 int pf_batch_commit(pf_batch* batch);
 /* Enqueue `launches` step launches; each advances every active job by its
- * steps per launch (one, or two: pf_batch_set_launch_steps), and a job stops
+ * steps per launch (one to three: pf_batch_set_launch_steps), and a job stops
  * at its target.  With launches_per_graph > 1 the launches are replayed from a
  * captured hipGraph of that many launches.  Asynchronous. */
 int pf_batch_run(pf_batch* batch, int launches, int launches_per_graph);

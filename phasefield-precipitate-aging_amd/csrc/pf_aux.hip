@@ -417,49 +417,71 @@ template hipError_t launch_summarize<float>(int, int, const float*, const float*
 // g_a(x_a) = 1/2 mu.A_a.mu, so sum_a p_a g_a(x_a) = 1/2 mu.(M mu) = 1/2 mu.r,
 // r = x - sum_a p_a xe_a.  Neighbours of the gradients go through the
 // boundary map (no-flux: the MMSP Neumann ghost copy; periodic: wrap).
+//
+// The sum is bound by the loads it issues, so a wave marches down a strip as
+// the step does (62 output columns, x neighbours by DPP, rows above and below
+// in registers): four loads per cell, three rows ahead, where a thread per cell
+// takes twelve.  3000^2 FP64: 78 -> 50 us (5.7 TB/s).
 template <typename T, int BC>
 __global__ __launch_bounds__(256) void energy_partial_kernel(
     const T* __restrict__ xCr, const T* __restrict__ xNb, const T* __restrict__ pd,
     const T* __restrict__ pl, int nx, int ny, EnergyParams E, double* __restrict__ chem_out,
-    double* __restrict__ grad_out, double* partials) {
+    double* __restrict__ grad_out, double* partials, int strips, int chunks, int rows) {
   const int Nx = nx - 2, Ny = ny - 2;
-  // a contiguous band of cells per XCD in each stride of the grid, so that the
-  // rows above and below mostly come from its own L2 (bound by the traffic of
-  // the neighbour rows: 3000^2 FP64 84 -> 78 us)
   const int block = xcd_remap(blockIdx.x, gridDim.x);
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wave = block * WPB + __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
   Kahan acc[2] = {};
   const double rx = 1.0 / (2.0 * E.dx), ry = 1.0 / (2.0 * E.dy);
-  for (Walk w(block, Nx); w.y < Ny; w.next()) {
-    const int x = w.x, y = w.y;
-    const size_t o = (size_t)(y + 1) * nx + (x + 1);
-    const double cr = (double)xCr[o] + E.xoff[0], nb = (double)xNb[o] + E.xoff[1];
-    const double fd = (double)pd[o], fl = (double)pl[o];
-    const double pD = p(fd), pL = p(fl), pG = 1.0 - pD - pL;
-    double mu0, mu1;
-    kks_mu(cr, nb, pD, pG, pL, mu0, mu1);
-    const double r0 = cr - pG * XE[0][0] - pD * XE[1][0] - pL * XE[2][0];
-    const double r1 = nb - pG * XE[0][1] - pD * XE[1][1] - pL * XE[2][1];
-    double g = 0.5 * (mu0 * r0 + mu1 * r1);
-    g += E.omega[0] * (fd * fd) * ((1.0 - fd) * (1.0 - fd));
-    g += E.omega[1] * (fl * fl) * ((1.0 - fl) * (1.0 - fl));
-    g += 2.0 * E.Omega * (fd * fd) * (fl * fl);
-    const size_t xl = (size_t)(y + 1) * nx + 1 + bc_map<BC>(x - 1, Nx);
-    const size_t xh = (size_t)(y + 1) * nx + 1 + bc_map<BC>(x + 1, Nx);
-    const size_t yl = (size_t)(1 + bc_map<BC>(y - 1, Ny)) * nx + (x + 1);
-    const size_t yh = (size_t)(1 + bc_map<BC>(y + 1, Ny)) * nx + (x + 1);
-    const T* phi[2] = {pd, pl};
-    double ge = 0.0;
+  for (int task = wave; task < strips * chunks; task += gridDim.x * WPB) {
+    const int gx = task % strips * STRIP + lane - 1;
+    const bool out_lane = lane >= 1 && lane <= STRIP && gx < Nx;
+    const int y0 = task / strips * rows, y1 = min(y0 + rows, Ny);
+    const uint32_t in_lane = (uint32_t)(1 + bc_map<BC>(gx, Nx)) * (uint32_t)sizeof(T);
+    // row y of the chunk in slot (y - y0 + 1) % RING: the window and three rows
+    // of loads; rows past the last one needed (y1) are that row again
+    constexpr int RING = 6;
+    Raw<T> ring[RING];
+    auto load = [&](Raw<T>& r, int y) {
+      const size_t row_b = (size_t)(1 + bc_map<BC>(min(y, y1), Ny)) * nx * sizeof(T);
+      load_row(r, xCr, xNb, pd, pl, row_b, in_lane);
+    };
 #pragma unroll
-    for (int k = 0; k < 2; k++) {
-      const double gx = ((double)phi[k][xh] - (double)phi[k][xl]) * rx;
-      const double gy = ((double)phi[k][yh] - (double)phi[k][yl]) * ry;
-      ge += E.kappa[k] * (gx * gx + gy * gy);
+    for (int k = 0; k < RING - 1; k++) load(ring[k], y0 - 1 + k);
+    for (int yb = y0; yb < y1; yb += RING) {
+#pragma unroll
+      for (int k = 0; k < RING; k++) {
+        const int y = yb + k;
+        if (y >= y1) break;
+        load(ring[(k + RING - 1) % RING], y + RING - 2);
+        const Raw<T>&S = ring[k], &C = ring[(k + 1) % RING], &N = ring[(k + 2) % RING];
+        const double cr = (double)C.cr + E.xoff[0], nb = (double)C.nb + E.xoff[1];
+        const double fd = (double)C.pd, fl = (double)C.pl;
+        const double pD = p(fd), pL = p(fl), pG = 1.0 - pD - pL;
+        double mu0, mu1;
+        kks_mu(cr, nb, pD, pG, pL, mu0, mu1);
+        const double r0 = cr - pG * XE[0][0] - pD * XE[1][0] - pL * XE[2][0];
+        const double r1 = nb - pG * XE[0][1] - pD * XE[1][1] - pL * XE[2][1];
+        double g = 0.5 * (mu0 * r0 + mu1 * r1);
+        g += E.omega[0] * (fd * fd) * ((1.0 - fd) * (1.0 - fd));
+        g += E.omega[1] * (fl * fl) * ((1.0 - fl) * (1.0 - fl));
+        g += 2.0 * E.Omega * (fd * fd) * (fl * fl);
+        const double gx0 = (from_right(fd) - from_left(fd)) * rx;
+        const double gx1 = (from_right(fl) - from_left(fl)) * rx;
+        const double gy0 = ((double)N.pd - (double)S.pd) * ry;
+        const double gy1 = ((double)N.pl - (double)S.pl) * ry;
+        double ge = E.kappa[0] * (gx0 * gx0 + gy0 * gy0);
+        ge += E.kappa[1] * (gx1 * gx1 + gy1 * gy1);
+        if (out_lane) {
+          const double c = g * E.dV, gg = ge * E.dV;
+          const size_t o = (size_t)(y + 1) * nx + (gx + 1);
+          if (chem_out) chem_out[o] = c;
+          if (grad_out) grad_out[o] = gg;
+          kadd(acc[0], c);
+          kadd(acc[1], gg);
+        }
+      }
     }
-    const double c = g * E.dV, gg = ge * E.dV;
-    if (chem_out) chem_out[o] = c;
-    if (grad_out) grad_out[o] = gg;
-    kadd(acc[0], c);
-    kadd(acc[1], gg);
   }
   __shared__ Kahan sh[2][256];
   for (int k = 0; k < 2; k++) sh[k][threadIdx.x] = acc[k];
@@ -495,16 +517,22 @@ template <typename T>
 hipError_t launch_energy(int nx, int ny, int bc, const EnergyParams& E, const T* xCr,
                          const T* xNb, const T* pd, const T* pl, double* chem, double* grad,
                          double* out3, const Scratch& S, hipStream_t st) {
-  const long N = (long)(nx - 2) * (ny - 2);
-  int blocks = (int)((N + 255) / 256);
-  if (blocks > REDUCE_BLOCKS) blocks = REDUCE_BLOCKS;
-  if (blocks < 1) blocks = 1;
+  // the shortest chunks whose waves are all resident at once, in one block's
+  // partial each (more only where the strips alone are that many)
+  const int Nx = nx - 2, Ny = ny - 2;
+  constexpr int MOST = REDUCE_BLOCKS * WPB;
+  const int strips = (Nx + STRIP - 1) / STRIP;
+  const int most_chunks = strips < MOST ? MOST / strips : 1;
+  const int rows = (Ny + most_chunks - 1) / most_chunks;
+  const int chunks = (Ny + rows - 1) / rows;
+  const long waves = (long)strips * chunks;
+  const int blocks = waves < MOST ? (int)((waves + WPB - 1) / WPB) : REDUCE_BLOCKS;
   if (bc == 0)
     hipLaunchKernelGGL((energy_partial_kernel<T, 0>), dim3(blocks), dim3(256), 0, st, xCr, xNb,
-                       pd, pl, nx, ny, E, chem, grad, S.partials);
+                       pd, pl, nx, ny, E, chem, grad, S.partials, strips, chunks, rows);
   else
     hipLaunchKernelGGL((energy_partial_kernel<T, 1>), dim3(blocks), dim3(256), 0, st, xCr, xNb,
-                       pd, pl, nx, ny, E, chem, grad, S.partials);
+                       pd, pl, nx, ny, E, chem, grad, S.partials, strips, chunks, rows);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(energy_final_kernel, dim3(1), dim3(128), 0, st, S.partials, blocks, out3);

@@ -543,8 +543,9 @@ __device__ __forceinline__ void march(
 // level l-1's rows y0-K+t-l-1 .. y0-K+t-l+1, the last of which level l-1 has
 // just produced.  Level l starts at iteration 2l, so the chunk reads old rows
 // y0-K .. y1-1+K and level l covers rows y0-(K-l) .. y1-1+(K-l).  Each level
-// keeps a three-row window in registers, row computed at iteration t in slot
-// t % 3; the first 2K iterations (the prologue) are unrolled at compile time.
+// keeps a window of rows in registers, the row computed at iteration t in slot
+// t % SLOTS; the first 2K iterations (the prologue) are unrolled at compile
+// time.
 //
 // With a window array `lw` in LDS (LW = true, the four-step kernel), each
 // level's centre row goes to LDS at the end of an iteration and comes back at
@@ -650,7 +651,7 @@ __device__ __forceinline__ void marchk_impl(
     quiet_rows = qr ? quiet_rows + 1 : 0;
   };
 
-  // windows: level l (0 = old fields) row of iteration t in slot t % 3
+  // windows: level l (0 = old fields) row of iteration t in slot t % SLOTS
   Point win[K][SLOTS];
   Centre cen[K][SLOTS];
   Raw<T> ring[DEPTH];

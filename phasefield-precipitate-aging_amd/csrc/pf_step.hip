@@ -120,12 +120,13 @@ __global__ __launch_bounds__(WAVE * WPB) void stepk_kernel(
 }
 
 // Four steps: the rows behind of the four levels' windows live in LDS (8 KiB
-// per wave, 32 KiB per block of WPB = 4 waves); 223 VGPRs allow two waves per
-// SIMD and the register budget is set to match.  At three waves per SIMD (168
-// VGPRs) it spills and takes twice as long.  FP64 4096^2: 326 us per launch
-// on a domain full of particles (380 us before the sums of update_cell were
-// nested and its constant addends kept in vector registers), 75% of it VALU
-// issue.
+// per wave, 32 KiB per block of WPB = 4 waves); 231-247 VGPRs allow two waves
+// per SIMD and the register budget is set to match.  At three waves per SIMD
+// (168 VGPRs) it spills and takes twice as long.  FP64 4096^2, us per launch: on
+// a domain full of particles 324-334, bound by FP64 issue (380 before the sums
+// of update_cell were nested and its constant addends kept in vector registers);
+// without precipitates 269 at 4.3 TB/s, bound by its 1.17 GB of traffic (331
+// before the modes, MODE_ROWS).
 template <typename T, int BC, int DEPTH, bool MODES, Mask MASK = FIVE, bool FAIR = false>
 __global__ __launch_bounds__(WAVE * WPB) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void step4_kernel(const T* __restrict__ iCr, const T* __restrict__ iNb,

@@ -40,8 +40,9 @@ def iter_launches(t0, n, max_steps, nuc_every=0):
 
 
 # FP32 storage: four steps per launch below this many interior cells, three
-# from it on (the four-step kernel is 5-15% faster at 1024^2-2048^2 and 3-4%
-# slower at 3072^2-8192^2, where the FP32 kernels are bound by arithmetic)
+# from it on (where every cell takes the full step, the four-step kernel is
+# 5-15% faster at 1024^2-2048^2 and 3-4% slower at 3072^2-8192^2: there the FP32
+# kernels are bound by arithmetic)
 FP32_FOUR_STEP_CELLS = 2560 * 2560
 
 
