@@ -245,9 +245,9 @@ static int rows4_model(int strips, int Ny) {
 
 // Chunks of this height and more run the march with modes (matrix and quiet
 // rows apart, pf_march.h).  Its 2K+1 dense rows at a chunk's start and three
-// times the code do not pay on short chunks (17 rows, 1400 x 1100 FP32: 39.5
-// against 36.7 us per four-step launch; 2 rows, 256^2: 10.5 against 8.8).
-// From here on, us per launch without / with modes:
+// times the code do not pay on short chunks (2 rows, 256^2: 10.5 against 8.8 us
+// per launch) unless the waves share their SIMDs fairly (fair_shares).  From
+// here on, us per launch without / with modes:
 //   FP64 4096^2, 75 rows, four steps: no precipitate 300 / 265, one particle's
 //   tail over the domain 314 / 282, particles everywhere 324 / 328;
 //   FP64 2048^2, 38 rows: 80.0 / 65.6, 86.5 / 88.3 with particles everywhere;
@@ -256,14 +256,25 @@ constexpr int MODE_ROWS = 32;
 
 // Whether the four-step launch shares its SIMDs fairly (FAIR, pf_march.h): where
 // all of it is resident at once, two waves on most SIMDs, and the chunks are
-// long enough to be cut in quarters.  us per launch without / with: 1400 x 1100
-// FP32, 14 rows, 36.7 / 34.6; FP64 1021 x 1543, 15 rows, 40.0 / 39.3; 1600 x
-// 1300, 21 rows, 47.9 / 46.8; 2048 x 1536, 28 rows, 65.7 / 64.5.  With later
-// rounds the waves are staggered anyway and the rule holds the old ones back
-// (4096^2, 60 rows: 329 / 357), and on chunks of one trip it holds back the
-// prologues (700^2, 6 rows: 17.9 / 18.9).
-static bool fair_shares(long waves, int rows) {
-  return waves > 1024 && waves <= 2048 && rows >= 12;
+// long enough to be cut in quarters.  The launch then ends with its slowest
+// wave, and where a domain has both matrix and precipitates the modes make
+// waves differ more, so the two go together.  us per launch with four
+// particles in the domain / particles everywhere, FAIR without modes, modes
+// without FAIR, both:
+//   FP64 2048 x 1536, 28 rows: 59.3 / 65.4, 49.7 / 70.2, 49.0 / 66.1;
+//   FP64 1700 x 1500, 23 rows: 51.2 / 56.5, 45.5 / 58.8, 44.3 / 57.6;
+//   FP64 1021 x 1543, 15 rows: 38.2 / 39.3, 35.5 / 42.7, 35.5 / 41.1;
+//   FP32 1800 x 1450, 24 rows: 52.9 / 53.5, 43.7 / 59.4, 41.1 / 57.6;
+//   FP32 1400 x 1100, 14 rows: 35.9 / 36.8, 33.1 / 39.8, 31.5 / 38.1.
+// FP32 takes it on long chunks too (2048^2, 38 rows: 67.5 / 86.5 with modes
+// alone, 65.8 / 81.2; 2400 x 2300, 49 rows: 79.2 / 108.4, 76.2 / 101.6); FP64,
+// nearer its traffic there and with some registers spilled, does not (2048^2:
+// 71.5 / 88.7, 79.5 / 86.6).  With later rounds the waves are staggered anyway
+// and the rule holds the old ones back (4096^2, 60 rows: 329 / 357), and on
+// chunks of one trip it holds back the prologues (700^2, 6 rows: 17.9 / 18.9).
+static bool fair_shares(long waves, int rows, int storage_bytes) {
+  return waves > 1024 && waves <= 2048 && rows >= 12 &&
+         (storage_bytes == 4 || rows < MODE_ROWS);
 }
 
 int default_rows_k(int k, int nx, int ny, int storage_bytes) {
@@ -322,10 +333,10 @@ static hipError_t launch_stepk_t(int nx, int ny, const StepParams& P, const T* i
 #undef PF_LAUNCH_TILE
       return hipGetLastError();
     }
-    if (rows >= MODE_ROWS)
+    if (fair_shares((long)strips * chunks, rows, (int)sizeof(T)))
+      PF_LAUNCH_MARCH((step4_kernel<T, BC, 3, true, FIVE, true>));
+    else if (rows >= MODE_ROWS)
       PF_LAUNCH_MARCH((step4_kernel<T, BC, 4, true>));
-    else if (DEPTH == 3 && fair_shares((long)strips * chunks, rows))
-      PF_LAUNCH_MARCH((step4_kernel<T, BC, 3, false, FIVE, true>));
     else
       PF_LAUNCH_MARCH((step4_kernel<T, BC, DEPTH, false>));
   } else if constexpr (K == 3 && sizeof(T) == sizeof(float)) {
