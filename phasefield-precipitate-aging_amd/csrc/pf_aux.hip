@@ -65,7 +65,8 @@ NucParams make_nuc(double sigma_del, double sigma_lav, double unit_a, double dx,
 // driving force times TINY is far below one.  In matrix cells mu = H_g (x - xe_g),
 // so a step changes it by at most |H_g| |q| |lap(mu)|.  False for NaN.
 static bool matrix_bounds(const StepParams& P) {
-  const double lm = fabs(P.m[1]) + fabs(P.m[7]) + fabs(P.m[3]) + fabs(P.m[5]) + fabs(P.m[4]);
+  double lm = 0.0;
+  for (int i = 0; i < 9; i++) lm += fabs(P.m[i]);
   const double h = fmax(fabs(H[0][0]) + fabs(H[0][1]), fabs(H[0][1]) + fabs(H[0][2]));
   const double q = fmax(fabs(P.qCr[0]) + fabs(P.qCr[1]), fabs(P.qNb[0]) + fabs(P.qNb[1]));
   const double qs = fmax(fabs(P.qs[0]), fabs(P.qs[1]));
@@ -78,7 +79,7 @@ static bool matrix_bounds(const StepParams& P) {
     if (!(G < 0x1p50) || !(fabs(P.c[a]) < 0x1p50) || !(fabs(P.k[a]) * lm + fabs(P.w[a]) < 14.0))
       return false;
   }
-  return symmetric_five_point(P.m);
+  return symmetric_five_point(P.m) || symmetric_nine_point(P.m);
 }
 
 StepParams make_step(double dt, const double* DCr, const double* DNb, const double* kappa,

@@ -610,7 +610,7 @@ __device__ __forceinline__ void marchk_impl(
     T* __restrict__ opl, int Nx, int Ny, int pitch, int strip, int chunk, int rows,
     const StepParams& P, LdsPtr lw) {
   static_assert(K >= 2 && K <= 4, "two to four steps per pass");
-  static_assert(MASK == FIVE || (MASK == NINE && !MODES), "symmetric masks; modes for FIVE");
+  static_assert(MASK == FIVE || MASK == NINE, "symmetric masks");
   // window rows in registers.  Two live rows suffice with the rows behind in
   // LDS; the plain march still rotates three names over six rows, which the
   // register allocator handles best, while the march with modes, three times

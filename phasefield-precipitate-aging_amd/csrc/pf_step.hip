@@ -253,6 +253,13 @@ static int rows4_model(int strips, int Ny) {
 //   FP64 2048^2, 38 rows: 80.0 / 65.6, 86.5 / 88.3 with particles everywhere;
 //   FP32 8192^2, 48 rows, three steps: 790 / 567, 802 / 818.
 constexpr int MODE_ROWS = 32;
+// The same for nine-point masks, whose rows cost more.  us per four-step launch
+// with four particles in the domain / particles everywhere, without, then with
+// modes: FP64 1021 x 1543, 15 rows: 42.3 / 45.0, 40.6 / 46.5; 2048 x 1536, 28
+// rows: 67.1 / 73.9, 53.8 / 76.8; 2000^2, 37 rows: 82.0 / 89.7, 65.6 / 92.9.
+// FP32 shares its SIMDs fairly besides, where fair_shares says so (2000^2: 82.8
+// / 83.1, 64.0 / 88.7, 62.0 / 84.8); in FP64 that spills (2000^2: 89.5 / 102.5).
+constexpr int NINE_MODE_ROWS = 20;
 
 // Whether the four-step launch shares its SIMDs fairly (FAIR, pf_march.h): where
 // all of it is resident at once, two waves on most SIMDs, and the chunks are
@@ -309,10 +316,17 @@ static hipError_t launch_stepk_t(int nx, int ny, const StepParams& P, const T* i
                      oNb, opd, opl, Nx, Ny, nx, strips, chunks, rows, remap, P)
   if constexpr (K != 3) {
     if (!folded_five_point(P.m)) {
-      if constexpr (K == 4)
-        PF_LAUNCH_MARCH((step4_kernel<T, BC, 3, false, NINE>));
-      else
+      if constexpr (K == 4) {
+        constexpr bool F32 = sizeof(T) == sizeof(float);
+        if (rows < NINE_MODE_ROWS)
+          PF_LAUNCH_MARCH((step4_kernel<T, BC, 3, false, NINE>));
+        else if (F32 && fair_shares((long)strips * chunks, rows, (int)sizeof(T)))
+          PF_LAUNCH_MARCH((step4_kernel<T, BC, F32 ? 3 : 4, true, NINE, F32>));
+        else
+          PF_LAUNCH_MARCH((step4_kernel<T, BC, 4, true, NINE>));
+      } else {
         PF_LAUNCH_MARCH((stepk_kernel<T, BC, K, 3, false, NINE>));
+      }
       return hipGetLastError();
     }
   }
