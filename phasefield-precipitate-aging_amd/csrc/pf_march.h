@@ -584,7 +584,7 @@ __device__ __forceinline__ void march(
 //    potentials exchanged.
 //  - DENSE: the general case, at the cost of the test (seven operations per
 //    row of some 430).
-// With FAIR, a wave's priority falls by quarters of its chunk.  The older of
+// With FAIR, a wave's priority within its SIMD falls by quarters of its chunk.  The older of
 // the two waves of a SIMD otherwise wins every issue slot, ends early and
 // leaves the other to run alone at two thirds of the pair's rate.
 //
