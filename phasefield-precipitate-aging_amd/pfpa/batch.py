@@ -6,6 +6,7 @@ import ctypes
 import numpy as np
 
 from ._lib import PfError, PfParams, check, lib
+from .hostmem import read_back
 from .model import LATTICE_CONST, SIGMA
 
 PF_STORAGE_F64 = 0
@@ -102,6 +103,7 @@ class Batch:
         check(blib().pf_batch_create(ctypes.byref(h), storage, int(pool_bytes), max_jobs),
               "pf_batch_create")
         self.h = h
+        read_back.open(h.value)
         self.shapes = {}
         self.offsets = {}
         self.launch_steps = 1
@@ -170,7 +172,7 @@ class Batch:
         """A job's current fields; compositions absolute (as FP64 when the job
         has an offset) unless `stored`."""
         ny, nx = self.shapes[jid]
-        out = [np.empty((ny, nx), dtype=self.dtype) for _ in range(4)]
+        out = [read_back.array((ny, nx), self.dtype) for _ in range(4)]
         check(blib().pf_batch_read(self.h, jid, *[a.ctypes.data_as(_vp) for a in out]),
               "pf_batch_read")
         off = self.offsets.get(jid, (0.0, 0.0))
@@ -214,6 +216,7 @@ class Batch:
 
     def close(self):
         if self.h is not None:
+            read_back.close(self.h.value)
             blib().pf_batch_destroy(self.h)
             self.h = None
 
