@@ -16,7 +16,8 @@ namespace pf {
 // x' = x + dt D lap(x_g) (src/discretization.cu:859-863) is
 //   x_Cr' = x_Cr + qCr[0] lap(mu0) + qCr[1] lap(mu1) + qs[0]
 // with dt (D_CrCr x_g,Cr + D_CrNb x_g,Nb) = qCr[0] mu0 + qCr[1] mu1 + qCr[2],
-// and likewise for Nb; qs = q[2] lap(1) is zero for a mask that sums to zero.
+// and likewise for Nb; qs = q[2] lap(1) is zero for a mask that sums to zero
+// within the rounding of its entries.
 // The Allen-Cahn update (src/discretization.cu:888-942) is
 //   phi' = phi + u (G(mu) u + w (2 phi - 1)) - c phi phi_o^2 + k lap(phi)
 // with u = phi (1 - phi), p'(phi) = 30 u^2, phi (phi - 1)(2 phi - 1) = -u (2 phi - 1)
