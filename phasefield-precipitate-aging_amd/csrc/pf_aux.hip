@@ -67,10 +67,11 @@ NucParams make_nuc(double sigma_del, double sigma_lav, double unit_a, double dx,
 static bool matrix_bounds(const StepParams& P) {
   double lm = 0.0;
   for (int i = 0; i < 9; i++) lm += fabs(P.m[i]);
-  const double h = fmax(fabs(H[0][0]) + fabs(H[0][1]), fabs(H[0][1]) + fabs(H[0][2]));
-  const double q = fmax(fabs(P.qCr[0]) + fabs(P.qCr[1]), fabs(P.qNb[0]) + fabs(P.qNb[1]));
-  const double qs = fmax(fabs(P.qs[0]), fabs(P.qs[1]));
-  double mu = h * (X_MATRIX + 1.0 + fmax(fabs(P.xoff[0]), fabs(P.xoff[1])));
+  // sums where the larger would do: fmax drops a NaN
+  const double h = fabs(H[0][0]) + 2.0 * fabs(H[0][1]) + fabs(H[0][2]);
+  const double q = fabs(P.qCr[0]) + fabs(P.qCr[1]) + fabs(P.qNb[0]) + fabs(P.qNb[1]);
+  const double qs = fabs(P.qs[0]) + fabs(P.qs[1]);
+  double mu = h * (X_MATRIX + 1.0 + fabs(P.xoff[0]) + fabs(P.xoff[1]));
   for (int step = 0; step < 4; step++) mu = 1.01 * (mu + h * (q * lm * mu + qs + 1e-5));
   for (int a = 0; a < 2; a++) {
     const double* g = P.g[a];
