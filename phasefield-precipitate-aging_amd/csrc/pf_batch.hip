@@ -15,10 +15,11 @@
 // three steps this launch, pf::march for one), then, if any job of the mix has
 // nucleation, the nucleation kernel (jobs whose schedule is due on the last
 // step of the launch; centre-only embeds).  The last block to finish, of the
-// step kernel or of a nucleation kernel with work to do, advances every active job's step counter, retires jobs that
-// reached their target and decides each job's next advance.  A job advances k steps in a launch (k up to the batch's steps per
-// launch) when k steps remain and no nucleation step falls before the last of
-// them.
+// step kernel or of a nucleation kernel with work to do, advances every active
+// job's step counter, retires jobs that reached their target and decides each
+// job's next advance.  A job advances k steps in a launch (k up to the batch's
+// steps per launch) when k steps remain and no nucleation step falls before the
+// last of them.
 // A job's arithmetic and tiling depend only on the job, so its result is the
 // same bits alone or in any mix.
 #include <hip/hip_runtime.h>
@@ -33,27 +34,34 @@
 
 namespace pf {
 
+// A job as the host sets it up; no kernel writes it.
 struct BatchJob {
   uint64_t off[2];       // element offsets of buffer sets 0 and 1 in the pool
   uint64_t plane;        // elements per field plane
-  uint64_t step;         // steps done
   uint64_t target;       // steps to run
   int Nx, Ny, pitch, bc;
   int strips, chunks, rows, wave0;
-  int active;            // 1 while step < target
   int nuc_every;         // 0 = no nucleation
-  int parity;            // buffer set holding the current fields
-  int adv;               // steps this launch advances the job (1, 2 or 3)
   int max_adv;           // steps per launch of the batch (1 where the grid is too small)
   int held;              // 1: the job takes no waves and does not advance (pf_batch_hold)
   StepParams P;
   NucParams N;
 };
 
+// How far a job is: read by every block of a launch, written by its last one.
+// Apart from BatchJob, whose reads the kernels may take for invariant (scalar
+// loads, also after stores).
+struct alignas(16) BatchState {
+  int active;            // 1 while step < target
+  int parity;            // buffer set holding the current fields
+  int adv;               // steps this launch advances the job (1, 2 or 3)
+  int pad;
+  uint64_t step;         // steps done
+};
+
 struct BatchHeader {
   int total_waves;
   int njobs;
-  unsigned int pad;
   unsigned int nuc_counters[4];  // [0] deferred events, [1] overflow flag, [2] wide events
   int any_due;                   // some active job has a nucleation step in this launch
   // per-XCD task counters of the step kernel (element [x][0]; zero between
@@ -68,25 +76,25 @@ struct BatchHeader {
 };
 
 // the last step of this launch is one of the job's nucleation steps
-__host__ __device__ __forceinline__ bool nuc_due(const BatchJob& J) {
-  return J.active && !J.held && J.nuc_every > 0 &&
-         (J.step + (uint64_t)J.adv - 1) % (uint64_t)J.nuc_every == 0;
+__host__ __device__ __forceinline__ bool nuc_due(const BatchJob& J, const BatchState& S) {
+  return S.active && !J.held && J.nuc_every > 0 &&
+         (S.step + (uint64_t)S.adv - 1) % (uint64_t)J.nuc_every == 0;
 }
 
 // the job's advance in the next launch (a multi-step launch never has a
 // nucleation step before its last step)
-__host__ __device__ __forceinline__ int next_adv(const BatchJob& J) {
+__host__ __device__ __forceinline__ int next_adv(const BatchJob& J, const BatchState& S) {
   int k = 1;
-  while (k < J.max_adv && J.step + k + 1 <= J.target &&
-         !(J.nuc_every > 0 && (J.step + k - 1) % (uint64_t)J.nuc_every == 0))
+  while (k < J.max_adv && S.step + k + 1 <= J.target &&
+         !(J.nuc_every > 0 && (S.step + k - 1) % (uint64_t)J.nuc_every == 0))
     k++;
   return k;
 }
 
 // Whether the calling block is the kernel's last to get here (the grid is a
 // multiple of 8 blocks).  The count needs no fence (one by each block writes
-// back its XCD's L2: 30 us per launch): a block has used every job entry and
-// task claim it read when it counts itself, the entries are written by no one
+// back its XCD's L2: 30 us per launch): a block has used every job state and
+// task claim it read when it counts itself, the states are written by no one
 // before, and the next launch sees what the last block writes.  Eight counters
 // first: a thousand atomics on one took 14 us.
 __device__ __forceinline__ bool last_block(BatchHeader* hdr) {
@@ -112,16 +120,19 @@ __device__ __forceinline__ bool last_block(BatchHeader* hdr) {
 // decide its next advance, and record whether any job is due at the next
 // launch.  (As a kernel of one block after the others this cost 4.5 us and a
 // gap per launch beside 50-90 us of steps.)
-__device__ __forceinline__ void advance_jobs(BatchJob* jobs, BatchHeader* hdr) {
+__device__ __forceinline__ void advance_jobs(const BatchJob* __restrict__ jobs,
+                                             BatchState* state, BatchHeader* hdr) {
   int due = 0;
   for (int j = threadIdx.x; j < hdr->njobs; j += blockDim.x) {
-    BatchJob& J = jobs[j];
-    if (J.active && !J.held) {
-      J.step += J.adv;
-      J.parity ^= 1;
-      if (J.step >= J.target) J.active = 0;
-      J.adv = next_adv(J);
-      due |= nuc_due(J) ? 1 : 0;
+    const BatchJob& J = jobs[j];
+    BatchState S = state[j];
+    if (S.active && !J.held) {
+      S.step += S.adv;
+      S.parity ^= 1;
+      if (S.step >= J.target) S.active = 0;
+      S.adv = next_adv(J, S);
+      state[j] = S;
+      due |= nuc_due(J, S) ? 1 : 0;
     }
   }
   due = __syncthreads_or(due);
@@ -129,6 +140,18 @@ __device__ __forceinline__ void advance_jobs(BatchJob* jobs, BatchHeader* hdr) {
     hdr->any_due = due;
     hdr->nuc_now = 0;
   }
+}
+
+// A job's state into scalar registers (all lanes read the same one).
+__device__ __forceinline__ BatchState uniform(const BatchState& S) {
+  BatchState u;
+  u.active = __builtin_amdgcn_readfirstlane(S.active);
+  u.parity = __builtin_amdgcn_readfirstlane(S.parity);
+  u.adv = __builtin_amdgcn_readfirstlane(S.adv);
+  u.pad = 0;
+  u.step = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)S.step) |
+           (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(S.step >> 32)) << 32;
+  return u;
 }
 
 constexpr int BATCH_RB = 16;  // reduction blocks per job
@@ -152,14 +175,13 @@ __device__ __forceinline__ void xcd_range(int total, int& first, int& last, int&
 // claims its next task from the XCD's counter (one atomic, by lane 0), so
 // waves that draw short tasks take more of them.  The claim for the next
 // task is issued before the current task runs and read after it; waves with
-// no first task leave the counter alone.  `table` is `jobs`, for the last
-// block to write.
+// no first task leave the counter alone.
 template <typename T, int DEPTH>
 __global__ __launch_bounds__(WAVE * WPB) void batch_step_kernel(const BatchJob* __restrict__ jobs,
                                                                 const int* __restrict__ wave_job,
                                                                 BatchHeader* __restrict__ hdr,
                                                                 T* __restrict__ pool,
-                                                                BatchJob* table) {
+                                                                BatchState* state) {
   int first, last, nwaves, w;
   xcd_range(hdr->total_waves, first, last, nwaves, w);
   unsigned int* ctr = &hdr->next_task[blockIdx.x & 7][0];
@@ -171,22 +193,23 @@ __global__ __launch_bounds__(WAVE * WPB) void batch_step_kernel(const BatchJob* 
     if (lane0) next = atomicAdd(ctr, 1u);
     const int j = __builtin_amdgcn_readfirstlane(wave_job[w]);
     const BatchJob& J = jobs[j];
-    if (!J.active) {
+    const BatchState st = uniform(state[j]);
+    if (!st.active) {
       w = first + nwaves + (int)__builtin_amdgcn_readfirstlane(next);
       continue;
     }
     const int local = w - J.wave0;
     const int strip = local % J.strips, chunk = local / J.strips;
-    const int par = J.parity;
+    const int par = st.parity;
     const T* in = pool + J.off[par];
     T* out = pool + J.off[par ^ 1];
     const uint64_t pl = J.plane;
 #define PF_BATCH_MARCH(BCV)                                                                  \
-  if (J.adv == 3)                                                                            \
+  if (st.adv == 3)                                                                           \
     marchk<T, BCV, 3, DEPTH, STRIP3>(in, in + pl, in + 2 * pl, in + 3 * pl, out, out + pl,     \
                                      out + 2 * pl, out + 3 * pl, J.Nx, J.Ny, J.pitch, strip,   \
                                      chunk, J.rows, J.P);                                      \
-  else if (J.adv == 2)                                                                       \
+  else if (st.adv == 2)                                                                      \
     marchk<T, BCV, 2, DEPTH, STRIP3>(in, in + pl, in + 2 * pl, in + 3 * pl, out, out + pl,     \
                                      out + 2 * pl, out + 3 * pl, J.Nx, J.Ny, J.pitch, strip,   \
                                      chunk, J.rows, J.P);                                      \
@@ -207,7 +230,7 @@ __global__ __launch_bounds__(WAVE * WPB) void batch_step_kernel(const BatchJob* 
   if (hdr->any_due) {  // the nucleation kernel comes first
     if (threadIdx.x == 0) hdr->nuc_now = 1;
   } else {
-    advance_jobs(table, hdr);
+    advance_jobs(jobs, state, hdr);
   }
 }
 
@@ -215,8 +238,8 @@ __global__ __launch_bounds__(WAVE * WPB) void batch_step_kernel(const BatchJob* 
 // step of this launch (src/main.cpp:307-316 schedule, centre-only embeds).
 template <typename T>
 __global__ __launch_bounds__(WAVE * WPB) void batch_nuc_kernel(
-    BatchJob* __restrict__ jobs, const int* __restrict__ wave_job, BatchHeader* __restrict__ hdr,
-    T* __restrict__ pool) {
+    const BatchJob* __restrict__ jobs, const int* __restrict__ wave_job,
+    BatchHeader* __restrict__ hdr, T* __restrict__ pool, BatchState* state) {
   int first, last, stride, w;
   xcd_range(hdr->total_waves, first, last, stride, w);
   const int lane = threadIdx.x & (WAVE - 1);
@@ -226,13 +249,14 @@ __global__ __launch_bounds__(WAVE * WPB) void batch_nuc_kernel(
   for (; w < last; w += stride) {
     const int j = __builtin_amdgcn_readfirstlane(wave_job[w]);
     const BatchJob& J = jobs[j];
-    const uint64_t s_last = J.step + J.adv - 1;  // the step whose output this is
-    if (!nuc_due(J)) continue;
+    const BatchState st = uniform(state[j]);
+    const uint64_t s_last = st.step + st.adv - 1;  // the step whose output this is
+    if (!nuc_due(J, st)) continue;
     const int local = w - J.wave0;
     const int strip = local % J.strips, chunk = local / J.strips;
     const int gx = strip * STRIP3 + lane - 1;
     if (lane < 1 || lane > STRIP3 || gx >= J.Nx) continue;
-    T* out = pool + J.off[J.parity ^ 1];
+    T* out = pool + J.off[st.parity ^ 1];
     const uint64_t pl = J.plane;
     NucParams N = J.N;
     N.call = s_last / (uint64_t)J.nuc_every;
@@ -260,7 +284,7 @@ __global__ __launch_bounds__(WAVE * WPB) void batch_nuc_kernel(
       }
     }
   }
-  if (last_block(hdr)) advance_jobs(jobs, hdr);
+  if (last_block(hdr)) advance_jobs(jobs, state, hdr);
 }
 
 // per-job deterministic compensated sums: block (j, r) reduces rows
@@ -283,13 +307,14 @@ __device__ __forceinline__ void kb_merge(KahanB& a, const KahanB& b) {
 
 template <typename T>
 __global__ __launch_bounds__(256) void batch_partial_kernel(const BatchJob* __restrict__ jobs,
+                                                            const BatchState* __restrict__ state,
                                                             const T* __restrict__ pool,
                                                             double* __restrict__ partials,
                                                             int job) {
   const BatchJob& J = jobs[job];
   const int r = blockIdx.x;
   const int ya = (int)(((long)J.Ny * r) / BATCH_RB), yb = (int)(((long)J.Ny * (r + 1)) / BATCH_RB);
-  const T* f = pool + J.off[J.parity];
+  const T* f = pool + J.off[state[job].parity];
   const uint64_t pl = J.plane;
   KahanB acc[5] = {};
   const long n = (long)(yb - ya) * J.Nx;
@@ -340,6 +365,7 @@ struct pf_batch {
   int max_jobs = 0;
   int max_waves = 0;
   pf::BatchJob* d_jobs = nullptr;
+  pf::BatchState* d_state = nullptr;
   int* d_wave_job = nullptr;
   pf::BatchHeader* d_hdr = nullptr;
   double* d_partials = nullptr;
@@ -351,6 +377,7 @@ struct pf_batch {
   int launch_steps = 1;  // steps per launch (1, 2 or 3)
   // host mirror
   std::vector<pf::BatchJob> jobs;       // slot -> job (slots are reused)
+  std::vector<pf::BatchState> state;    // slot -> how far it is
   std::vector<int> slot_live;           // 1 if the slot holds a job
   std::vector<int> slot_on_device;      // 1 if the device table holds the slot's current job
   std::map<uint64_t, uint64_t> free_;   // offset -> size (elements)
@@ -418,16 +445,12 @@ int sync_jobs_from_device(pf_batch* b) {
   hipError_t e = hipStreamSynchronize(b->stream);
   if (e != hipSuccess) return bhip(e, "batch synchronize");
   if (b->jobs.empty()) return PF_OK;
-  std::vector<pf::BatchJob> dev(b->jobs.size());
-  e = hipMemcpy(dev.data(), b->d_jobs, dev.size() * sizeof(pf::BatchJob), hipMemcpyDeviceToHost);
-  if (e != hipSuccess) return bhip(e, "read job table");
+  std::vector<pf::BatchState> dev(b->jobs.size());
+  e = hipMemcpy(dev.data(), b->d_state, dev.size() * sizeof(pf::BatchState),
+                hipMemcpyDeviceToHost);
+  if (e != hipSuccess) return bhip(e, "read job states");
   for (size_t j = 0; j < dev.size(); j++)
-    if (b->slot_live[j] && b->slot_on_device[j]) {
-      b->jobs[j].step = dev[j].step;
-      b->jobs[j].active = dev[j].active;
-      b->jobs[j].parity = dev[j].parity;
-      b->jobs[j].adv = dev[j].adv;
-    }
+    if (b->slot_live[j] && b->slot_on_device[j]) b->state[j] = dev[j];
   return PF_OK;
 }
 
@@ -438,21 +461,21 @@ hipError_t launch_batch_step(pf_batch* b, hipStream_t st) {
   switch (b->depth) {
     case 2:
       hipLaunchKernelGGL((pf::batch_step_kernel<T, 2>), grid, block, 0, st, b->d_jobs,
-                         b->d_wave_job, b->d_hdr, pool, b->d_jobs);
+                         b->d_wave_job, b->d_hdr, pool, b->d_state);
       break;
     case 6:
       hipLaunchKernelGGL((pf::batch_step_kernel<T, 6>), grid, block, 0, st, b->d_jobs,
-                         b->d_wave_job, b->d_hdr, pool, b->d_jobs);
+                         b->d_wave_job, b->d_hdr, pool, b->d_state);
       break;
     default:
       hipLaunchKernelGGL((pf::batch_step_kernel<T, 3>), grid, block, 0, st, b->d_jobs,
-                         b->d_wave_job, b->d_hdr, pool, b->d_jobs);
+                         b->d_wave_job, b->d_hdr, pool, b->d_state);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || !b->nuc) return e;
   // a quarter of the blocks: nearly every launch only looks at one flag
   hipLaunchKernelGGL(pf::batch_nuc_kernel<T>, dim3(b->grid_blocks / 32 * 8), block, 0, st,
-                     b->d_jobs, b->d_wave_job, b->d_hdr, pool);
+                     b->d_jobs, b->d_wave_job, b->d_hdr, pool, b->d_state);
   return hipGetLastError();
 }
 
@@ -493,6 +516,8 @@ int pf_batch_create(pf_batch** out, int storage, size_t pool_bytes, int max_jobs
   hipError_t e;
   if ((e = hipMalloc(&b->pool, b->pool_elems * b->elem)) != hipSuccess ||
       (e = hipMalloc((void**)&b->d_jobs, (size_t)max_jobs * sizeof(pf::BatchJob))) != hipSuccess ||
+      (e = hipMalloc((void**)&b->d_state, (size_t)max_jobs * sizeof(pf::BatchState))) !=
+          hipSuccess ||
       (e = hipMalloc((void**)&b->d_wave_job, (size_t)b->max_waves * sizeof(int))) != hipSuccess ||
       (e = hipMalloc((void**)&b->d_hdr, sizeof(pf::BatchHeader))) != hipSuccess ||
       (e = hipMalloc((void**)&b->d_partials, pf::BATCH_RB * 10 * sizeof(double))) != hipSuccess ||
@@ -523,6 +548,7 @@ void pf_batch_destroy(pf_batch* b) {
   if (b->graph) (void)hipGraphExecDestroy(b->graph);
   if (b->pool) (void)hipFree(b->pool);
   if (b->d_jobs) (void)hipFree(b->d_jobs);
+  if (b->d_state) (void)hipFree(b->d_state);
   if (b->d_wave_job) (void)hipFree(b->d_wave_job);
   if (b->d_hdr) (void)hipFree(b->d_hdr);
   if (b->d_partials) (void)hipFree(b->d_partials);
@@ -598,6 +624,7 @@ int pf_batch_add(pf_batch* b, const pf_job_desc* d, const void* xCr, const void*
     if ((int)b->jobs.size() >= b->max_jobs) return bfail(PF_ERR_ARG, "job table full");
     slot = (int)b->jobs.size();
     b->jobs.emplace_back();
+    b->state.emplace_back();
     b->slot_live.push_back(0);
     b->slot_on_device.push_back(0);
   }
@@ -608,14 +635,11 @@ int pf_batch_add(pf_batch* b, const pf_job_desc* d, const void* xCr, const void*
   J.plane = n / 8;
   J.off[0] = off;
   J.off[1] = off + 4 * J.plane;
-  J.step = 0;
-  J.parity = 0;
   J.target = d->steps;
   J.Nx = d->Nx;
   J.Ny = d->Ny;
   J.pitch = d->Nx + 2;
   J.bc = d->bc;
-  J.active = d->steps > 0 ? 1 : 0;
   J.nuc_every = d->nucleation ? d->nuc_every : 0;
   J.P = pf::make_step(d->prm.dt, d->prm.DCr, d->prm.DNb, d->prm.kappa, d->prm.omega,
                       d->prm.Lmob, d->prm.alpha, d->prm.mask, d->x_offset);
@@ -638,6 +662,7 @@ int pf_batch_add(pf_batch* b, const pf_job_desc* d, const void* xCr, const void*
   e = hipStreamSynchronize(b->upload);
   if (e != hipSuccess) return bhip(e, "upload job fields");
   b->jobs[slot] = J;
+  b->state[slot] = pf::BatchState{d->steps > 0 ? 1 : 0, 0, 1, 0, 0};
   b->slot_live[slot] = 1;
   b->slot_on_device[slot] = 0;
   b->dirty = true;
@@ -652,7 +677,7 @@ int pf_batch_remove(pf_batch* b, int job_id) {
   if (int r = sync_jobs_from_device(b)) return r;
   pf::BatchJob& J = b->jobs[job_id];
   pool_free(b, J.off[0], 8 * J.plane);
-  J.active = 0;
+  b->state[job_id].active = 0;
   b->slot_live[job_id] = 0;
   b->slot_on_device[job_id] = 0;
   b->dirty = true;
@@ -666,8 +691,9 @@ int pf_batch_commit(pf_batch* b) {
   std::vector<int> wave_job;
   for (size_t j = 0; j < b->jobs.size(); j++) {
     pf::BatchJob& J = b->jobs[j];
+    pf::BatchState& S = b->state[j];
     if (!b->slot_live[j]) {
-      J.active = 0;
+      S.active = 0;
       J.wave0 = 0;
       J.strips = J.chunks = 0;
       continue;
@@ -676,9 +702,9 @@ int pf_batch_commit(pf_batch* b) {
     J.strips = (J.Nx + pf::STRIP3 - 1) / pf::STRIP3;
     J.chunks = (J.Ny + J.rows - 1) / J.rows;
     J.max_adv = (J.Nx >= 3 && J.Ny >= 3) ? b->launch_steps : 1;
-    J.adv = J.active ? pf::next_adv(J) : 1;
+    S.adv = S.active ? pf::next_adv(J, S) : 1;
     J.wave0 = (int)wave_job.size();
-    if (!J.active || J.held) {
+    if (!S.active || J.held) {
       J.wave0 = 0;
       continue;  // finished and held jobs take no waves
     }
@@ -691,6 +717,10 @@ int pf_batch_commit(pf_batch* b) {
       (e = hipMemcpy(b->d_jobs, b->jobs.data(), b->jobs.size() * sizeof(pf::BatchJob),
                      hipMemcpyHostToDevice)) != hipSuccess)
     return bhip(e, "upload job table");
+  if (!b->jobs.empty() &&
+      (e = hipMemcpy(b->d_state, b->state.data(), b->state.size() * sizeof(pf::BatchState),
+                     hipMemcpyHostToDevice)) != hipSuccess)
+    return bhip(e, "upload job states");
   if (!wave_job.empty() &&
       (e = hipMemcpy(b->d_wave_job, wave_job.data(), wave_job.size() * sizeof(int),
                      hipMemcpyHostToDevice)) != hipSuccess)
@@ -701,7 +731,6 @@ int pf_batch_commit(pf_batch* b) {
   h.total_waves = (int)wave_job.size();
   h.njobs = (int)b->jobs.size();
   for (int x = 0; x < 8; x++) h.next_task[x][0] = 0u;
-  h.pad = 0u;
   for (int x = 0; x < 8; x++) h.blocks_done[x][0] = 0u;
   h.groups_done = 0u;
   h.nuc_now = 0;
@@ -709,8 +738,8 @@ int pf_batch_commit(pf_batch* b) {
   b->nuc = false;
   for (size_t j = 0; j < b->jobs.size(); j++)
     if (b->slot_live[j]) {
-      if (pf::nuc_due(b->jobs[j])) h.any_due = 1;
-      if (b->jobs[j].active && !b->jobs[j].held && b->jobs[j].nuc_every > 0) b->nuc = true;
+      if (pf::nuc_due(b->jobs[j], b->state[j])) h.any_due = 1;
+      if (b->state[j].active && !b->jobs[j].held && b->jobs[j].nuc_every > 0) b->nuc = true;
     }
   if ((e = hipMemcpy(b->d_hdr, &h, sizeof(h), hipMemcpyHostToDevice)) != hipSuccess)
     return bhip(e, "upload header");
@@ -767,8 +796,8 @@ int pf_batch_poll(pf_batch* b, int job_id, uint64_t* steps_done, int* active) {
   if (job_id < 0 || job_id >= (int)b->jobs.size() || !b->slot_live[job_id])
     return bfail(PF_ERR_ARG, "no such job");
   if (int r = sync_jobs_from_device(b)) return r;
-  if (steps_done) *steps_done = b->jobs[job_id].step;
-  if (active) *active = b->jobs[job_id].active;
+  if (steps_done) *steps_done = b->state[job_id].step;
+  if (active) *active = b->state[job_id].active;
   return PF_OK;
 }
 
@@ -781,8 +810,8 @@ int pf_batch_poll_all(pf_batch* b, int capacity, int* job_ids, uint64_t* steps_d
     if (!b->slot_live[j]) continue;
     if (n < capacity) {
       if (job_ids) job_ids[n] = (int)j;
-      if (steps_done) steps_done[n] = b->jobs[j].step;
-      if (active) active[n] = b->jobs[j].active;
+      if (steps_done) steps_done[n] = b->state[j].step;
+      if (active) active[n] = b->state[j].active;
     }
     n++;
   }
@@ -798,7 +827,7 @@ int pf_batch_read(pf_batch* b, int job_id, void* xCr, void* xNb, void* pd, void*
   const pf::BatchJob& J = b->jobs[job_id];
   const size_t bytes = (size_t)(J.Nx + 2) * (J.Ny + 2) * b->elem;
   void* dst[4] = {xCr, xNb, pd, pl};
-  const char* base = (const char*)b->pool + J.off[J.parity] * b->elem;
+  const char* base = (const char*)b->pool + J.off[b->state[job_id].parity] * b->elem;
   for (int k = 0; k < 4; k++) {
     if (!dst[k]) continue;
     hipError_t e = hipMemcpy(dst[k], base + k * J.plane * b->elem, bytes, hipMemcpyDeviceToHost);
@@ -815,10 +844,10 @@ int pf_batch_summarize(pf_batch* b, int job_id, double* out5) {
   if (int r = sync_jobs_from_device(b)) return r;
   if (b->storage == PF_STORAGE_F32)
     hipLaunchKernelGGL(pf::batch_partial_kernel<float>, dim3(pf::BATCH_RB), dim3(256), 0,
-                       b->stream, b->d_jobs, (const float*)b->pool, b->d_partials, job_id);
+                       b->stream, b->d_jobs, b->d_state, (const float*)b->pool, b->d_partials, job_id);
   else
     hipLaunchKernelGGL(pf::batch_partial_kernel<double>, dim3(pf::BATCH_RB), dim3(256), 0,
-                       b->stream, b->d_jobs, (const double*)b->pool, b->d_partials, job_id);
+                       b->stream, b->d_jobs, b->d_state, (const double*)b->pool, b->d_partials, job_id);
   hipLaunchKernelGGL(pf::batch_final_kernel, dim3(1), dim3(64), 0, b->stream, b->d_jobs,
                      b->d_partials, job_id, b->d_out5);
   hipError_t e = hipGetLastError();
@@ -861,7 +890,7 @@ int pf_batch_waves(pf_batch* b) {
   if (!b) return 0;
   int total = 0;
   for (size_t j = 0; j < b->jobs.size(); j++)
-    if (b->slot_live[j] && b->jobs[j].active && !b->jobs[j].held)
+    if (b->slot_live[j] && b->state[j].active && !b->jobs[j].held)
       total += ((b->jobs[j].Nx + pf::STRIP3 - 1) / pf::STRIP3) *
                ((b->jobs[j].Ny + b->rows - 1) / b->rows);
   return total;

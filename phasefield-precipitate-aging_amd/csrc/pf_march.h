@@ -38,7 +38,6 @@ namespace pf {
 
 constexpr int WAVE = 64;
 constexpr int STRIP = WAVE - 2;   // output columns per strip
-constexpr int STRIP2 = WAVE - 4;  // output columns per strip of the two-step march
 constexpr int STRIP3 = WAVE - 6;  // and of the three-step march (the batched form's strips)
 constexpr int WPB = 4;           // waves (strips) per block: adjacent strips of one row chunk
 constexpr int UNROLL = 6;        // multiple of the 3-row window and of every ring depth
