@@ -159,6 +159,12 @@ int pf_advance_f32(pf_ctx* ctx, int nx, int ny, int bc, const pf_params* prm,
                    float* const* a, float* const* b, uint64_t steps, int steps_per_launch,
                    int* in_b, void* stream);
 
+/* Steps of the first launch pf_advance_* makes for `steps` steps with this mask
+ * (nine weights) and grid: most = steps_per_launch, or fewer where the mask, the
+ * grid or the steps left do not take that many.  0 for 0 steps, a null mask or
+ * a `most` that is not 1 to 4. */
+int pf_launch_steps(int nx, int ny, const double* mask, uint64_t steps, int most);
+
 /* Standalone nucleation pass in place on the given fields.  Replaces
  * device_nucleation (src/discretization.cu:1179-1209). */
 int pf_nucleation_f64(pf_ctx* ctx, int nx, int ny, double* conc_Cr, double* conc_Nb,

@@ -137,8 +137,18 @@ int stepk_t(int k, pf_ctx* ctx, int nx, int ny, int bc, const pf_params* prm, co
   return PF_OK;
 }
 
-// `steps` plain steps from set a, alternating between the sets, up to `most`
-// per launch where the mask and the grid take multi-step launches.
+// Steps of the next launch of pf_advance_* with `steps` left: `most` of them
+// where the mask and the grid take that many per launch.
+int launch_steps(int nx, int ny, const double* mask, uint64_t steps, int most) {
+  const bool five = pf::symmetric_five_point(mask);
+  const bool nine = !five && pf::symmetric_nine_point(mask);
+  if (!(five || nine) || nx < 5 || ny < 5) most = 1;
+  if (most == 4 && (nx < 6 || ny < 6)) most = 3;
+  const int k = steps < (uint64_t)most ? (int)steps : most;
+  return nine && k == 3 ? 2 : k;  // no three-step kernel takes nine points
+}
+
+// `steps` plain steps from set a, alternating between the sets.
 template <typename T>
 int advance_t(pf_ctx* ctx, int nx, int ny, int bc, const pf_params* prm, T* const* a,
               T* const* b, uint64_t steps, int most, int* in_b, void* stream) {
@@ -153,16 +163,11 @@ int advance_t(pf_ctx* ctx, int nx, int ny, int bc, const pf_params* prm, T* cons
   if (int r = check_disjoint<T>(nx, ny, b[0], b[1], b[2], b[3], a[0], a[1], a[2], a[3])) return r;
   const pf::StepParams P = pf::make_step(prm->dt, prm->DCr, prm->DNb, prm->kappa, prm->omega,
                                          prm->Lmob, prm->alpha, prm->mask, storage_offset<T>(ctx));
-  const bool five = pf::symmetric_five_point(prm->mask);
-  const bool nine = !five && pf::symmetric_nine_point(prm->mask);
-  if (!(five || nine) || nx < 5 || ny < 5) most = 1;
-  if (most == 4 && (nx < 6 || ny < 6)) most = 3;
   hipStream_t st = (hipStream_t)stream;
   int flip = 0;
   *in_b = 0;
   while (steps > 0) {
-    int k = steps < (uint64_t)most ? (int)steps : most;
-    if (nine && k == 3) k = 2;
+    const int k = launch_steps(nx, ny, prm->mask, steps, most);
     T* const* i = flip ? b : a;
     T* const* o = flip ? a : b;
     const hipError_t e =
@@ -376,6 +381,11 @@ int pf_advance_f32(pf_ctx* ctx, int nx, int ny, int bc, const pf_params* prm, fl
                    float* const* b, uint64_t steps, int steps_per_launch, int* in_b,
                    void* stream) {
   return advance_t<float>(ctx, nx, ny, bc, prm, a, b, steps, steps_per_launch, in_b, stream);
+}
+
+int pf_launch_steps(int nx, int ny, const double* mask, uint64_t steps, int most) {
+  if (!mask || most < 1 || most > 4) return 0;
+  return launch_steps(nx, ny, mask, steps, most);
 }
 
 int pf_step_loop_f64(pf_ctx* ctx, int n, const pf_step_item* items, void* stream) {

@@ -72,6 +72,7 @@ PROTOTYPES = {
                             ctypes.POINTER(_vp), ctypes.c_uint64, _i, ctypes.POINTER(_i), _vp]),
     "pf_advance_f32": (_i, [_vp, _i, _i, _i, ctypes.POINTER(PfParams), ctypes.POINTER(_vp),
                             ctypes.POINTER(_vp), ctypes.c_uint64, _i, ctypes.POINTER(_i), _vp]),
+    "pf_launch_steps": (_i, [_i, _i, ctypes.POINTER(ctypes.c_double), ctypes.c_uint64, _i]),
     "pf_ctx_set_tile2": (_i, [_vp, _i, _i]),
     "pf_default_rows2": (_i, [_i, _i, _i]),
     "pf_ctx_set_tile3": (_i, [_vp, _i, _i]),

@@ -1,8 +1,8 @@
-"""Native stepping loop over the C-ABI.  The steps between two nucleation
-steps are one call (pf_advance_*), which runs up to four per launch (the
-temporally blocked kernels); nucleation steps, the ones the reference's schedule selects
-(kernel_time % nuc_interval == 0, src/main.cpp:307-316), run one per launch
-with the nucleation pass fused."""
+"""Native stepping loop over the C-ABI.  The steps between two nucleation steps
+are one call (pf_advance_*), which runs up to four per launch (the temporally
+blocked kernels); nucleation steps, the ones the reference's schedule selects
+(kernel_time % nuc_interval == 0, src/main.cpp:307-316), run one per launch with
+the nucleation pass fused."""
 import ctypes
 
 import numpy as np
@@ -17,26 +17,34 @@ def _ptr(t):
     return ctypes.c_void_p(t.data_ptr())
 
 
-def iter_launches(t0, n, max_steps, nuc_every=0):
-    """Launches that advance steps t0 .. t0+n-1, one (k, nucleation) at a
-    time with k steps per launch.  A launch groups up to `max_steps` steps
-    none of which is a nucleation step (t % nuc_every == 0,
-    src/main.cpp:307-316); a nucleation step runs alone with the nucleation
-    pass (nucleation True).  nuc_every 0 = nucleation off.  O(1) per launch,
-    so a stepping loop can start launching at once."""
+def segments(t0, n, nuc_every=0):
+    """Native calls that advance steps t0 .. t0+n-1, one (k, nucleation) at a
+    time: a nucleation step (t % nuc_every == 0, src/main.cpp:307-316) alone
+    with the nucleation pass, the k steps up to the next one (or the end) in one
+    pf_advance_* call.  nuc_every 0 = nucleation off."""
     t, end = t0, t0 + n
     while t < end:
-        if nuc_every > 0:
-            nxt = -(-t // nuc_every) * nuc_every  # first nucleation step >= t
-            if nxt == t:
-                yield (1, True)
-                t += 1
-                continue
-            k = min(max_steps, end - t, nxt - t)
+        if nuc_every > 0 and t % nuc_every == 0:
+            k, nucleate = 1, True
         else:
-            k = min(max_steps, end - t)
-        yield (k, False)
+            k = end - t if nuc_every <= 0 else min(end - t, nuc_every - t % nuc_every)
+            nucleate = False
+        yield k, nucleate
         t += k
+
+
+def iter_launches(t0, n, max_steps, nuc_every=0, nx=1 << 10, ny=1 << 10, mask=None):
+    """Launches of Simulation.step for steps t0 .. t0+n-1, one (k, nucleation)
+    at a time with k steps per launch, up to `max_steps`, as pf_advance_* groups
+    them for this mask and grid (by default ones that take any number)."""
+    weights = (ctypes.c_double * 9)(*(mask or M.five_point_mask(1.0, 1.0)))
+    for steps, nucleate in segments(t0, n, nuc_every):
+        while steps > 0:
+            k = 1 if nucleate else lib().pf_launch_steps(nx, ny, weights, steps, max_steps)
+            if k < 1:
+                raise ValueError("steps per launch must be 1, 2, 3 or 4")
+            yield k, nucleate
+            steps -= k
 
 
 # FP32 storage: four steps per launch below this many interior cells, three
@@ -66,7 +74,7 @@ def default_steps_per_launch(setup, dtype, requested=None):
 
 
 def plan_launches(t0, n, max_steps, nuc_every=0):
-    """iter_launches as a list."""
+    """iter_launches as a list (five-point mask, a large grid)."""
     return list(iter_launches(t0, n, max_steps, nuc_every))
 
 
@@ -232,30 +240,25 @@ class Simulation:
 
     def step(self, n=1):
         st = ctypes.c_void_p(self.stream.cuda_stream)
-        end = self.steps_done + n
-        while self.steps_done < end:
+        every = self.nuc_every if self.nucleation else 0
+        for k, nucleate in segments(self.steps_done, n, every):
             a, b = self.a, self.b
-            t = self.steps_done
-            if self.nucleation and t % self.nuc_every == 0:
-                self.N.call = t // self.nuc_every
+            if nucleate:
+                self.N.call = self.steps_done // self.nuc_every
                 check(self._step(self.ctx, self.nx, self.ny, self.s.bc, ctypes.byref(self.P),
                                  _ptr(a[0]), _ptr(a[1]), _ptr(a[2]), _ptr(a[3]),
                                  _ptr(b[0]), _ptr(b[1]), _ptr(b[2]), _ptr(b[3]),
                                  ctypes.byref(self.N), st), "pf_step")
-                self.a, self.b = b, a
-                self.steps_done += 1
-                continue
-            # the steps up to the next nucleation step in one native call
-            k = end - t
-            if self.nucleation:
-                k = min(k, self.nuc_every - t % self.nuc_every)
-            in_b = ctypes.c_int()
-            most = 4 if self._group_other_masks else self.steps_per_launch
-            check(self._advance(self.ctx, self.nx, self.ny, self.s.bc, ctypes.byref(self.P),
-                                (ctypes.c_void_p * 4)(*[x.data_ptr() for x in a]),
-                                (ctypes.c_void_p * 4)(*[x.data_ptr() for x in b]), k,
-                                most, ctypes.byref(in_b), st), "pf_advance")
-            if in_b.value:
+                flipped = True
+            else:
+                in_b = ctypes.c_int()
+                most = 4 if self._group_other_masks else self.steps_per_launch
+                check(self._advance(self.ctx, self.nx, self.ny, self.s.bc, ctypes.byref(self.P),
+                                    (ctypes.c_void_p * 4)(*[x.data_ptr() for x in a]),
+                                    (ctypes.c_void_p * 4)(*[x.data_ptr() for x in b]), k,
+                                    most, ctypes.byref(in_b), st), "pf_advance")
+                flipped = in_b.value
+            if flipped:
                 self.a, self.b = b, a
             self.steps_done += k
 
