@@ -239,9 +239,13 @@ class Simulation:
         return best, times
 
     def step(self, n=1):
+        """Advance n steps (any whole number, numpy's types included)."""
+        if n != int(n):
+            raise ValueError("a whole number of steps")
+        n = int(n)
         st = ctypes.c_void_p(self.stream.cuda_stream)
         every = self.nuc_every if self.nucleation else 0
-        for k, nucleate in segments(self.steps_done, n, every):
+        for k, nucleate in segments(int(self.steps_done), n, int(every)):
             a, b = self.a, self.b
             if nucleate:
                 self.N.call = self.steps_done // self.nuc_every
