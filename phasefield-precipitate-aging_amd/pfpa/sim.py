@@ -55,12 +55,12 @@ FP32_FOUR_STEP_CELLS = 2560 * 2560
 
 
 def default_steps_per_launch(setup, dtype, requested=None):
-    """Steps per launch of a Simulation: `requested` (1 to 4), or by default
-    the faster kernel on the grids measured: four for FP64 storage, and for
-    FP32 four below FP32_FOUR_STEP_CELLS interior cells and three above;
-    reduced to what the grid and mask allow: the multi-step kernels take
-    symmetric five-point masks and an interior of at least 3x3 (four steps:
-    4x4)."""
+    """Steps per launch of a Simulation by the pf_step2..4_* entry points, which
+    take symmetric five-point masks: `requested` (1 to 4), or by default the
+    faster kernel on the grids measured: four for FP64 storage, and for FP32
+    four below FP32_FOUR_STEP_CELLS interior cells and three above; reduced to
+    what the grid allows, an interior of at least 3x3 (four steps: 4x4).  1 for
+    other masks; Simulation.launch_steps tells what those run."""
     if requested is None:
         cells = (setup.nx - 2) * (setup.ny - 2)
         requested = 4 if dtype == torch.float64 or cells < FP32_FOUR_STEP_CELLS else 3
@@ -165,11 +165,21 @@ class Simulation:
                        4: lib().pf_step4_f64 if f64 else lib().pf_step4_f32}
         self._advance = lib().pf_advance_f64 if f64 else lib().pf_advance_f32
         self.steps_per_launch = default_steps_per_launch(setup, dtype, steps_per_launch)
-        # other masks have no pf_step2..4_* entry points, but symmetric
-        # nine-point ones run four steps per launch all the same (pf_advance_*)
-        self._group_other_masks = (steps_per_launch is None and
-                                   not M.symmetric_five_point(setup.mask))
+        # other masks have no pf_step2..4_* entry points, but pf_advance_* runs
+        # symmetric nine-point ones several steps per launch all the same: as
+        # many as asked for, four by default
+        self._other_masks = None
+        if not M.symmetric_five_point(setup.mask):
+            self._other_masks = 4 if steps_per_launch is None else steps_per_launch
         self._summ = lib().pf_summarize_f64 if dtype == torch.float64 else lib().pf_summarize_f32
+
+    @property
+    def launch_steps(self):
+        """The most steps step() runs in one launch: steps_per_launch for
+        symmetric five-point masks; for symmetric nine-point ones the steps per
+        launch asked for (two where that is three), four by default; else 1."""
+        most = self.steps_per_launch if self._other_masks is None else self._other_masks
+        return lib().pf_launch_steps(self.nx, self.ny, self.P.mask, 4, most)
 
     def set_tile(self, rows, remap=1, depth=0):
         check(lib().pf_ctx_set_tile(self.ctx, rows, remap, depth), "pf_ctx_set_tile")
@@ -256,7 +266,7 @@ class Simulation:
                 flipped = True
             else:
                 in_b = ctypes.c_int()
-                most = 4 if self._group_other_masks else self.steps_per_launch
+                most = self.steps_per_launch if self._other_masks is None else self._other_masks
                 check(self._advance(self.ctx, self.nx, self.ny, self.s.bc, ctypes.byref(self.P),
                                     (ctypes.c_void_p * 4)(*[x.data_ptr() for x in a]),
                                     (ctypes.c_void_p * 4)(*[x.data_ptr() for x in b]), k,
