@@ -208,8 +208,10 @@ class Simulation:
         heuristic for two and three) are within a few per cent of the best on
         the grids measured; this measures the grid at hand.  rows_set None:
         the kernel's default height and 6, 8, 12, 16, 24, 32, 48, 60, 64, 72,
-        96 (those up to the interior height).  Results do not depend on the
-        tile.  Returns (rows, {rows: us per launch})."""
+        96 (those up to the interior height), and for four steps 0, which
+        leaves the choice to the launch: square tiles without chunks on a small
+        grid, else the default height.  Results do not depend on the tile.
+        Returns (rows, {rows: us per launch})."""
         k = self.steps_per_launch
         if k < 2:
             raise ValueError("tune_tile needs two or more steps per launch")
@@ -217,7 +219,7 @@ class Simulation:
             storage = 0 if self.dtype == torch.float64 else 1
             default = getattr(lib(), "pf_default_rows%d" % k)(self.nx, self.ny, storage)
             rows_set = sorted({default} | {r for r in (6, 8, 12, 16, 24, 32, 48, 60, 64, 72, 96)
-                                          if r <= self.ny - 2})
+                                          if r <= self.ny - 2} | ({0} if k == 4 else set()))
         fn = self._stepk[k]
         set_tile = {2: self.set_tile2, 3: self.set_tile3, 4: self.set_tile4}[k]
         st = ctypes.c_void_p(self.stream.cuda_stream)
