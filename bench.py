@@ -735,6 +735,29 @@ def trace_summary(path, last=200):
             sum(tail) / len(tail)))
 
 
+# Lists of single measurements whose best or extreme values the line holds beside them.
+DETAILS = ("table", "fp64_replays")
+
+
+def line(out):
+    """The result line: what the headline rests on in full, the further
+    sections' numbers to six digits and without their lists of single
+    measurements, which go to stderr (all in full were 21 KB, more than a
+    reader that keeps the last 16 KB of the output sees)."""
+    def short(v):
+        if isinstance(v, dict):
+            return {k: short(x) for k, x in v.items() if k not in DETAILS}
+        if isinstance(v, list):
+            return [short(x) for x in v]
+        return float("%.6g" % v) if isinstance(v, float) else v
+
+    sections = ("dropin", "mobility_divergence", "batched", "precision", "serving", "cpu_baseline")
+    for k in ("batched", "serving"):
+        if k in out:
+            log("%s, all: %s" % (k, json.dumps(out[k])))
+    return json.dumps({k: short(v) if k in sections else v for k, v in out.items()})
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -908,7 +931,7 @@ def main():
         log("cpu:", json.dumps(cpu))
     out["cpu_baseline"] = cpu
     out["bench_wall_s"] = time.perf_counter() - t_all
-    print(json.dumps(out))
+    print(line(out))
 
 
 if __name__ == "__main__":
