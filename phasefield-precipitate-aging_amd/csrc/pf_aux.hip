@@ -438,10 +438,11 @@ template hipError_t launch_summarize<float>(int, int, const float*, const float*
 // A gradient's division by 2 dx: a r with r = 1 / d rounded, corrected once by
 // its residual, is a / d rounded (Markstein 1990, barring under- and overflow),
 // for three operations; a plain division's dozen, four times a cell, cost 8 us.
-// Outside the range where no step of it can under- or overflow to any effect
-// (a smaller result's square is zero), and for infinities and NaN, the wave
-// divides.  3000^2 FP64, sum and reductions: 152.6 us with a r alone, 153.9 so,
-// 161.1 with divisions.
+// The wave divides where the spacings are so far out that a step of it could
+// under- or overflow to some effect (with spacings in the range a smaller
+// result's square is zero), or where the sum is not finite: overflow, infinities
+// and NaN all end there.  3000^2 FP64, sum and reductions: 154.3 us with a r
+// alone, 155.2 so, 161-163 with divisions.
 __device__ __forceinline__ double quotient(double a, double d, double r) {
   const double q = a * r;
   return fma(fma(-d, q, a), r, q);
@@ -498,16 +499,15 @@ __global__ __launch_bounds__(256) void energy_partial_kernel(
         g += 2.0 * E.Omega * (fd * fd) * (fl * fl);
         const double ax0 = from_right(fd) - from_left(fd), ax1 = from_right(fl) - from_left(fl);
         const double ay0 = (double)N.pd - (double)S.pd, ay1 = (double)N.pl - (double)S.pl;
-        double gx0, gx1, gy0, gy1;
-        if (regular && __all(fabs(ax0) + fabs(ax1) + fabs(ay0) + fabs(ay1) < 0x1p500)) {
-          gx0 = quotient(ax0, dx2, rx), gx1 = quotient(ax1, dx2, rx);
-          gy0 = quotient(ay0, dy2, ry), gy1 = quotient(ay1, dy2, ry);
-        } else {
-          gx0 = ax0 / dx2, gx1 = ax1 / dx2;
-          gy0 = ay0 / dy2, gy1 = ay1 / dy2;
-        }
-        double ge = E.kappa[0] * (gx0 * gx0 + gy0 * gy0);
-        ge += E.kappa[1] * (gx1 * gx1 + gy1 * gy1);
+        auto gradient = [&](double gx0, double gx1, double gy0, double gy1) {
+          double e = E.kappa[0] * (gx0 * gx0 + gy0 * gy0);
+          e += E.kappa[1] * (gx1 * gx1 + gy1 * gy1);
+          return e;
+        };
+        double ge = gradient(quotient(ax0, dx2, rx), quotient(ax1, dx2, rx),
+                             quotient(ay0, dy2, ry), quotient(ay1, dy2, ry));
+        if (!(regular && __all(fabs(ge) < HUGE_VAL)))
+          ge = gradient(ax0 / dx2, ax1 / dx2, ay0 / dy2, ay1 / dy2);
         if (out_lane) {
           const double c = g * E.dV, gg = ge * E.dV;
           const size_t o = (size_t)(y + 1) * nx + (gx + 1);
