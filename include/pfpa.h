@@ -281,8 +281,9 @@ int pf_default_rows(int nx, int ny);
  * heuristic) and prefetch depth (2, 3, 6; 0 = 3).  pf_default_rows2 (3, 4) is
  * its heuristic for storage PF_STORAGE_F64 or PF_STORAGE_F32.  Four steps (and
  * FP32 three) keep a depth of their own on tall chunks and where all of a
- * launch is resident at once, and so do nine-point masks; with rows = 0 four steps on a small grid run by square
- * tiles, without chunks.  The results do not depend on any of these. */
+ * launch is resident at once, whatever is set, and so do nine-point masks; with
+ * rows = 0 four steps on a small grid run by square tiles, without chunks.  The
+ * results do not depend on any of these. */
 int pf_ctx_set_tile2(pf_ctx* ctx, int rows, int depth);
 int pf_default_rows2(int nx, int ny, int storage);
 int pf_ctx_set_tile3(pf_ctx* ctx, int rows, int depth);

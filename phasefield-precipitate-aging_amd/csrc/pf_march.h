@@ -374,7 +374,8 @@ __device__ __forceinline__ void update_compositions(const StepParams& P, const A
   nNb = cc.xNb + fma(P.qNb[0], lap_mu[0], fma(P.qNb[1], lap_mu[1], ad.qs[1]));
 }
 __device__ __forceinline__ void update_cell(const StepParams& P, const Addends& ad,
-                                            const double lap[4], const Point& cur, const Centre& cc, double& nCr, double& nNb,
+                                            const double lap[4], const Point& cur,
+                                            const Centre& cc, double& nCr, double& nNb,
                                             double& npd, double& npl) {
   update_compositions(P, ad, lap + 2, cc, nCr, nNb);
   const double fd = cur.pd, fl = cur.pl;
@@ -588,9 +589,11 @@ __device__ __forceinline__ void march(
 //    potentials exchanged.
 //  - DENSE: the general case, at the cost of the test (seven operations per
 //    row of some 430).
-// With FAIR, a wave's priority within its SIMD falls by quarters of its chunk.  The older of
-// the two waves of a SIMD otherwise wins every issue slot, ends early and
-// leaves the other to run alone at two thirds of the pair's rate.
+// The rows of the prologue are dense or matrix; quiet ones begin behind it.
+//
+// With FAIR, a wave's priority within its SIMD falls by quarters of its chunk.
+// The older of the two waves of a SIMD otherwise wins every issue slot, ends
+// early and leaves the other to run alone at two thirds of the pair's rate.
 //
 // Every mode gives the bits of DENSE: StepParams::matrix_ok says (from bounds
 // on the coefficients) that a step multiplies |phi| < TINY by 16 at most, that

@@ -244,10 +244,10 @@ static int rows4_model(int strips, int Ny) {
 }
 
 // Chunks of this height and more run the march with modes (matrix and quiet
-// rows apart, pf_march.h).  Its 2K+1 dense rows at a chunk's start and three
-// times the code do not pay on short chunks (2 rows, 256^2: 10.5 against 8.8 us
-// per launch) unless the waves share their SIMDs fairly (fair_shares).  From
-// here on, us per launch without / with modes:
+// rows apart, pf_march.h).  The 2K rows of a chunk's prologue, which are dense or
+// matrix but never quiet, and three times the code do not pay on short chunks
+// (2 rows, 256^2: 10.5 against 8.8 us per launch) unless the waves share their
+// SIMDs fairly (fair_shares).  From here on, us per launch without / with modes:
 //   FP64 4096^2, 75 rows, four steps: no precipitate 300 / 265, one particle's
 //   tail over the domain 314 / 282, particles everywhere 324 / 328;
 //   FP64 2048^2, 38 rows: 80.0 / 65.6, 86.5 / 88.3 with particles everywhere;

@@ -48,9 +48,13 @@ def iter_launches(t0, n, max_steps, nuc_every=0, nx=1 << 10, ny=1 << 10, mask=No
 
 
 # FP32 storage: four steps per launch below this many interior cells, three
-# from it on (where every cell takes the full step, the four-step kernel is
-# 5-15% faster at 1024^2-2048^2 and 3-4% slower at 3072^2-8192^2: there the FP32
-# kernels are bound by arithmetic)
+# from it on.  The line was drawn where the two took the same time, with every
+# cell taking the full step.  Now that matrix and quiet rows are taken apart four
+# are as fast or faster beyond it too, us per step at three / four without
+# precipitates, then with particles everywhere: 2560^2 29.9 / 17.5, 30.0 / 29.9;
+# 3072^2 41.5 / 27.1, 41.7 / 42.1; 4096^2 56.1 / 45.7, 79.4 / 75.2; 8192^2 189.5 /
+# 167.2, 283.7 / 272.9.  The default has stayed where programs know it; a caller
+# asks for steps_per_launch=4.
 FP32_FOUR_STEP_CELLS = 2560 * 2560
 
 

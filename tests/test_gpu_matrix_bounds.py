@@ -50,9 +50,9 @@ def test_parameters_out_of_bounds_match_one_step_launches(gpu, k, dtype, nine, k
     Nx, Ny, bc = 130, 67, 1
     s = M.make_setup(Nx, Ny, bc=bc)
     rng = np.random.default_rng(17)
-    fields = [M.fill_ghosts(a, bc) for a in
-              (rng.uniform(0.28, 0.33, (Ny + 2, Nx + 2)), rng.uniform(0.02, 0.027, (Ny + 2, Nx + 2)))
-              + _phi(kind, Ny, Nx, rng)]
+    size = (Ny + 2, Nx + 2)
+    x = (rng.uniform(0.28, 0.33, size), rng.uniform(0.02, 0.027, size))
+    fields = [M.fill_ghosts(a, bc) for a in x + _phi(kind, Ny, Nx, rng)]
     mask = M.nine_point_mask(s.dx, s.dx) if nine else s.mask
     P = PfParams()
     P.dt, P.alpha = s.dt, s.alpha

@@ -10,7 +10,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("nucleation", [False, True])
-@pytest.mark.parametrize("n", [np.int64(9), np.int32(9), np.uint8(9), 9.0, np.float64(9), np.array(9)])
+@pytest.mark.parametrize("n", [np.int64(9), np.int32(9), np.uint8(9), 9.0, np.float64(9),
+                               np.array(9)])
 def test_types_of_a_count(gpu, n, nucleation):
     s = M.make_setup(40, 30, bc=1)
     f = M.init_matrix_with_particles(40, 30, s.dx, 1, seed=2, n_del=1, n_lav=0, radius=1e-9)

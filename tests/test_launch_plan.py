@@ -40,7 +40,9 @@ def test_refused():
 
 
 def test_plans_of_other_masks():
-    plan = lambda mask, n, most=4: [k for k, _ in iter_launches(0, n, most, 0, 100, 80, mask)]  # noqa: E731
+    def plan(mask, n, most=4):
+        return [k for k, _ in iter_launches(0, n, most, 0, 100, 80, mask)]
+
     assert plan(NINE, 11) == [4, 4, 2, 1] and plan(NINE, 7, 3) == [2, 2, 2, 1]
     assert plan(LOPSIDED, 3) == [1, 1, 1]
     assert list(iter_launches(0, 8, 4, 5, 100, 80, NINE)) == [(1, True), (4, False), (1, True),
