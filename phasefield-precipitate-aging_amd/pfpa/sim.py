@@ -37,7 +37,7 @@ def iter_launches(t0, n, max_steps, nuc_every=0, nx=1 << 10, ny=1 << 10, mask=No
     """Launches of Simulation.step for steps t0 .. t0+n-1, one (k, nucleation)
     at a time with k steps per launch, up to `max_steps`, as pf_advance_* groups
     them for this mask and grid (by default ones that take any number)."""
-    weights = (ctypes.c_double * 9)(*(mask or M.five_point_mask(1.0, 1.0)))
+    weights = (ctypes.c_double * 9)(*(M.five_point_mask(1.0, 1.0) if mask is None else mask))
     for steps, nucleate in segments(t0, n, nuc_every):
         while steps > 0:
             k = 1 if nucleate else lib().pf_launch_steps(nx, ny, weights, steps, max_steps)

@@ -55,3 +55,8 @@ def test_segments():
                                         (1, False)]
     assert list(segments(7, 2, 5)) == [(2, False)]
     assert list(segments(2, 3, 1)) == [(1, True)] * 3
+
+
+def test_a_mask_may_be_an_array():
+    import numpy as np
+    assert [k for k, _ in iter_launches(0, 5, 4, 0, 100, 80, np.array(NINE))] == [4, 1]
